@@ -223,12 +223,13 @@ enum tmx_option {
                                    their kernels are launched one by one (measured faster) */
   TMX_OPT_SWEEP_PAIRS = 17,     /* > 0: the elasticity finest level runs its first two
                                    pre-sweeps as one launch, in node-row chunks of this height
-                                   (default 8); 0: one launch per sweep */
+                                   (default at most 8, lower on small grids); 0: one launch per sweep */
   TMX_OPT_SWEEP_PAIRS_POST = 18, /* the same for prolongation with the first two post-sweeps
-                                   (default 12 for FP32 V-cycles, 16 for FP64) */
+                                   (default at most 12 for FP32 V-cycles, 16 for
+                                   FP64, lower on small grids) */
   TMX_OPT_SWEEP_PAIR_RESTRICT = 19, /* > 0: with two pre-sweeps, the zero-start pair also forms
                                    the residual and restricts it to the next level, in chunks
-                                   of this many rows (default 12); 0: a separate launch.
+                                   of this many rows (default at most 12); 0: a separate launch.
                                    Setting any of 17-19 applies to both precisions;
                                    tmx_autotune re-picks the heights of those left > 0 */
   TMX_OPT_FILTER_PIPE = 20,     /* > 0: the filter's finest level (even nx, ny; at most 4

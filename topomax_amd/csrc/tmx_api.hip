@@ -82,8 +82,12 @@ static int create_impl(const tmx_problem_desc* d, tmx_problem* h) {
   h->el.nu_coarse_ = 3;  // with Chebyshev steps a third coarse sweep pays for itself
   // the filter's band kernels make extra sweeps cheap: three on every level measured fastest
   h->fl.nu_pre_ = h->fl.nu_post_ = h->fl.nu_coarse_ = 3;
-  // FP64 element level 1 is faster launch per sweep: its band kernels are VALU-bound there
-  h->el.band_first_fp64_ = 2;
+  // A large FP64 element level 1 is faster launch per sweep (seven launches a visit): its band
+  // kernels are VALU-bound there; a small one is bound by its launches.  Whole FP64 steps, band
+  // kernels against launches per sweep: 300 x 100 cells on level 1 3132 / 3496 us, 600 x 200
+  // 3722 / 3951, 750 x 250 4826 / 5017, 900 x 300 5998 / 5864, 1200 x 400 6855 / 6700.
+  h->el.band_first_fp64_ =
+      h->el.levels_.size() > 1 && h->el.levels_[1].nn <= kBandFirstNodesFp64 ? 1 : 2;
   const size_t nv = (size_t)(h->nx + 1) * (h->ny + 1);
   TMX_TRY(h->F.alloc(2 * nv));
   TMX_TRY(h->Fm.alloc(2 * nv));
@@ -703,6 +707,8 @@ extern "C" int tmx_set_option(tmx_problem* h, int option, double value) {
         (option == TMX_OPT_SWEEP_PAIRS        ? h->el.pair_rows_
          : option == TMX_OPT_SWEEP_PAIRS_POST ? h->el.pair_rows_post_
                                               : h->el.pair_rr_rows_)[i] = (int)value;
+      if (option == TMX_OPT_SWEEP_PAIR_RESTRICT)
+        h->el.pair_rr_rows_merged_[0] = h->el.pair_rr_rows_merged_[1] = 0;
       break;
     case TMX_OPT_FINE_CELL_WEIGHTS:
       if (value < 0 || value > 3 || value != std::floor(value)) return invalid("mask must be 0..3");
@@ -810,6 +816,7 @@ extern "C" int tmx_autotune(tmx_problem* h, int* rows_out, double* best_us_out) 
                    : kind == 1 ? h->el.pair_rows_post_
                                : h->el.pair_rr_rows_)[prec == 0 ? 1 : 0];
       if (slot <= 0) continue;  // switched off by the caller
+      if (kind == 2) h->el.pair_rr_rows_merged_[prec == 0 ? 1 : 0] = 0;
       const int op1 = kind == 0 ? kSmoothZero : kProlongSmooth;
       auto launch = [&](int rows) -> int {
         if (kind == 2) {

@@ -94,6 +94,9 @@ constexpr int kRingBB = 24;
 // PCG slots (flag, rr, iters contiguous for one async read)
 constexpr PcgSlots kPcg = {10, 11, 16, 12, 13, 15, 14, 17, 18, 19};
 
+// largest FP64 elasticity level 1 (nodes) that runs the band kernels (tmx_problem_create)
+constexpr size_t kBandFirstNodesFp64 = 200000;
+
 enum LevelKind : int { kElem = 0, kStencil = 1, kDense = 2 };
 enum Phys : int { kElasticity = 0, kFilter = 1 };
 
@@ -304,11 +307,14 @@ class Hierarchy {
   int band_wide_ = 2;
   // > 0: the finest elasticity level's first two pre-sweeps (pair_rows_), and its prolongation
   // with the first two post-sweeps (pair_rows_post_), run as one launch each with node-row
-  // chunks of that height; 0: one launch per sweep.  Index 0: FP32 V-cycles, 1: FP64.
+  // chunks of that height; 0: one launch per sweep.  Index 0: FP32 V-cycles, 1: FP64.  init()
+  // lowers these heights (the upper ends) on small grids.
   int pair_rows_[2] = {8, 8}, pair_rows_post_[2] = {12, 16};
   // > 0: with two pre-sweeps, the zero-start pair also forms the residual and restricts it
   // (chunks of this many rows); 0: a separate residual + restriction launch
   int pair_rr_rows_[2] = {12, 12};
+  // the same inside a merged batch step (0: as alone); each node's result is the same
+  int pair_rr_rows_merged_[2] = {0, 0};
   // elasticity element levels 0 .. pair_levels_ - 1 use the paired column-strip kernels (the
   // coarser ones with chunk heights pair_rows_coarse_ [pre, post, fused restriction] and
   // pair_nu_coarse_ sweeps each way, 0: nu_coarse_); the levels below them the band kernels
