@@ -707,8 +707,6 @@ extern "C" int tmx_set_option(tmx_problem* h, int option, double value) {
         (option == TMX_OPT_SWEEP_PAIRS        ? h->el.pair_rows_
          : option == TMX_OPT_SWEEP_PAIRS_POST ? h->el.pair_rows_post_
                                               : h->el.pair_rr_rows_)[i] = (int)value;
-      if (option == TMX_OPT_SWEEP_PAIR_RESTRICT)
-        h->el.pair_rr_rows_merged_[0] = h->el.pair_rr_rows_merged_[1] = 0;
       break;
     case TMX_OPT_FINE_CELL_WEIGHTS:
       if (value < 0 || value > 3 || value != std::floor(value)) return invalid("mask must be 0..3");
@@ -816,7 +814,6 @@ extern "C" int tmx_autotune(tmx_problem* h, int* rows_out, double* best_us_out) 
                    : kind == 1 ? h->el.pair_rows_post_
                                : h->el.pair_rr_rows_)[prec == 0 ? 1 : 0];
       if (slot <= 0) continue;  // switched off by the caller
-      if (kind == 2) h->el.pair_rr_rows_merged_[prec == 0 ? 1 : 0] = 0;
       const int op1 = kind == 0 ? kSmoothZero : kProlongSmooth;
       auto launch = [&](int rows) -> int {
         if (kind == 2) {

@@ -313,8 +313,6 @@ class Hierarchy {
   // > 0: with two pre-sweeps, the zero-start pair also forms the residual and restricts it
   // (chunks of this many rows); 0: a separate residual + restriction launch
   int pair_rr_rows_[2] = {12, 12};
-  // the same inside a merged batch step (0: as alone); each node's result is the same
-  int pair_rr_rows_merged_[2] = {0, 0};
   // elasticity element levels 0 .. pair_levels_ - 1 use the paired column-strip kernels (the
   // coarser ones with chunk heights pair_rows_coarse_ [pre, post, fused restriction] and
   // pair_nu_coarse_ sweeps each way, 0: nu_coarse_); the levels below them the band kernels

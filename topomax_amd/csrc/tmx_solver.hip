@@ -119,17 +119,16 @@ int Hierarchy::init(Phys phys, int nx, int ny, double hx, double hy, unsigned fi
     // 2839 / 2830 / 2892 / 2941 / 3066, 1200 x 400 3911 / 3749 / 3622 / 3687 / 3642, 1800 x 600
     // 6697 / 6175 / 6116 / 6032 / 5866; mixed 600 x 200 2280 / 2306 / 2351 / 2379 / 2478,
     // 1200 x 400 3019 / 2932 / 2938 / 2965 / 3033, 1800 x 600 4546 / 4326 / 4299 / 4290 / 4305.
-    // FP64 chunks need about one wave per SIMD (104 registers), FP32 chunks two.  In a merged
+    // A design alone would take one wave per SIMD (FP64, 104 registers) or two; in a merged
     // batch step the other designs fill the chip and the halo rows are what counts: 32 designs
-    // of N 40-320 take 8389 us with 2048 waves a design, 7998 with 512 (the start's 12 rows:
-    // 8034).  The prolongation pair's chunks also set the order of the r.z partials, which a
-    // design alone and in a batch have to share, so they take the batch's line.
+    // of N 40-320 (mixed) take 8389 us with 2048 waves a design, 8199 with 1024, 7998 with 512
+    // and 8034 with 12 rows throughout.  Chunk boundaries order the sums at the last bit, and a
+    // design's results in a batch are those it has alone, so both take the same heights.
     for (int pk = 0; pk < 2; ++pk) {
-      const int waves = pk == 1 ? 1280 : 2048;
+      const int waves = pk == 1 ? 640 : 512;
       pair_rows_[pk] = pair_rows_for(nx, ny, 60, waves, 8);
       pair_rr_rows_[pk] = pair_rows_for(nx, ny, 56, waves, 12);
-      pair_rr_rows_merged_[pk] = pair_rows_for(nx, ny, 56, 512, 12);
-      pair_rows_post_[pk] = pair_rows_for(nx, ny, 60, pk == 1 ? 640 : 512, pk == 1 ? 16 : 12);
+      pair_rows_post_[pk] = pair_rows_for(nx, ny, 60, waves, pk == 1 ? 16 : 12);
     }
   }
   if (phys == kElasticity) {  // the overlapped coarse build's stream and events, made up front
@@ -780,10 +779,7 @@ int Hierarchy::vcycle(int l, const T* b, T* out, hipStream_t s, RedSlot* dot_bz)
   const int pi = sizeof(T) == 8 ? 1 : 0;
   const int rows_pre = l == 0 ? pair_rows_[pi] : pair_rows_coarse_[0];
   const int rows_post = l == 0 ? pair_rows_post_[pi] : pair_rows_coarse_[1];
-  const int rows_rr = l > 0 ? pair_rows_coarse_[2]
-                      : active_recorder() && pair_rr_rows_merged_[pi] > 0
-                          ? pair_rr_rows_merged_[pi]
-                          : pair_rr_rows_[pi];
+  const int rows_rr = l == 0 ? pair_rr_rows_[pi] : pair_rows_coarse_[2];
   const bool pair_pre = pair_level && rows_pre > 0 && npre >= 2;
   const bool pair_post = pair_level && rows_post > 0 && fused_el && npost >= 2;
   const bool pair_rr = pair_pre && npre == 2 && fused_el && rows_rr > 0;
