@@ -196,36 +196,47 @@ hipError_t stencil_rap(int nxf, int nyf, int nxc, int nyc, int nested, unsigned 
 template <int BS>
 hipError_t stencil_to_dense(int nx, int ny, const double* st, double* dense, hipStream_t s);
 
-// Bottom of a V-cycle in one workgroup of kTailThreads: 9-point levels lev[0..nlev-2]
-// (bilinear transfers, at most kTailThreads nodes each) and the dense coarsest lev[nlev-1]
-// (x = Ainv b).  Every level's vectors live in LDS (lev[l].off, in elements of T: iterate,
-// ping-pong and right-hand side, BS*nn each; the dense level holds b and x); b_in (global)
-// is the top level's right-hand side and x_out (global) receives its result.
+// Bottom of a V-cycle in one workgroup of kTailWg threads: levels lev[0..nlev-2] with explicit
+// 9-point rows (bilinear transfers, at most kTailNodes nodes on the top level and kTailWg on
+// those below) and the dense coarsest lev[nlev-1] (x = Ainv b, cn unknowns).  The caller gives each level's cells and rows; the
+// launcher fills in the LDS layout.  Every level's vectors live in LDS (from lev[l].off, in
+// elements of T: iterate and ping-pong with a border of zeros, `padded` each, then the
+// right-hand side; the dense level holds b and x); b_in (global) is the top level's right-hand
+// side and x_out (global) receives its result.
 constexpr int kMaxTail = 8;
-constexpr int kTailThreads = 1024;
-constexpr int kTailNodes = kTailThreads;
-constexpr size_t kTailLdsBytes = 64 * 1024;
+constexpr int kTailWg = 512;              // threads
+constexpr int kTailHelpers = 8;           // workgroups that read the rows into the L2
+constexpr int kTailNodes = 2 * kTailWg;   // nodes of the top level; kTailWg below it
+constexpr size_t kTailLdsBytes = 128 * 1024;  // the vectors
+constexpr size_t kTailLdsMax = 160 * 1024;    // with the coarsest inverse
+struct TailDims {
+  int nx, ny;
+};
 template <typename T>
 struct TailLevel {
   int nx, ny;
-  const T* st;  // 9-point stencil (global, SoA as for stencil_op)
-  int off;      // LDS offset of this level's vectors, in elements of T
+  const T* st;   // 9-point stencil (global, SoA as for stencil_op)
+  int off;       // LDS offset of this level's vectors, in elements of T
+  int padded;    // elements of one vector with its border
+  unsigned div;  // ceil(2^20 / (nx + 1))
 };
 constexpr int kMaxNu = 8;  // smoothing sweeps per pass in the tail kernel
 template <typename T>
 struct TailDesc {
   int nlev, cn, nu_pre, nu_post;
   unsigned fixed;
+  int zero;       // elements cleared at the start
+  int dense_off;  // > 0: LDS byte offset that the coarsest inverse is copied to
   T omega[kMaxNu];  // step size of sweep k of a smoothing pass
   const double* dense;
   const T* b_in;
   T* x_out;
   TailLevel<T> lev[kMaxTail];
 };
-// LDS bytes a tail over these levels needs (9-point levels nn[0..nlev-2], dense level nn[nlev-1])
-size_t tail_lds_bytes(const size_t* nn, int nlev, int bs, size_t elem);
+// LDS bytes of a tail's vectors over these levels (the last one dense)
+size_t tail_lds_bytes(const TailDims* lev, int nlev, int bs, size_t elem);
 template <typename T, int BS>
-hipError_t tail_vcycle(const TailDesc<T>& d, size_t lds_bytes, hipStream_t s);
+hipError_t tail_vcycle(const TailDesc<T>& d, hipStream_t s);
 hipError_t dense_invert(int n, double* a, double* work, hipStream_t s);
 template <typename T>
 hipError_t dense_apply(int n, const double* ainv, const T* b, T* x, hipStream_t s);

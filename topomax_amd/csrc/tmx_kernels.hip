@@ -2295,307 +2295,449 @@ TMX_INST_S9F(float, 1)
 TMX_INST_S9F(float, 2)
 
 // ---------------------------------------------------------------- tail V-cycle
-// The bottom of the hierarchy (9-point levels of at most kTailThreads nodes, then the dense
-// coarsest solve) runs as a single workgroup that steps through the whole V-cycle with a
-// barrier between steps: one launch instead of ~7 per level.  Vectors stay in LDS; each
-// thread owns one node and holds that node's stencil row in registers while its level is
-// being smoothed, so a sweep costs LDS traffic only.
+// The bottom of the hierarchy (levels with explicit 9-point rows of at most kTailNodes nodes,
+// then the dense coarsest solve) runs as a single workgroup that steps through the whole V-cycle
+// with a barrier between steps: one launch instead of ~7 per level.  It is bound by latency: one
+// CU, a chain of LDS round trips and barriers.  So each thread owns a node (or two) and holds its
+// row in registers while its level is smoothed; the vectors that neighbours read lie in LDS with
+// a border of zeros, so a row's nine neighbours are at fixed distances and the transfers need
+// no range checks; the 1-D transfer weights (0, 1/2, 1) follow from a node's parity; and steps that
+// touch only the thread's own node (restriction's result and the first sweep from zero) share a
+// phase.  Per V-cycle of 816 + 225 + 65 nodes and 42 coarsest unknowns, three sweeps each way
+// (N=1000): 18.5 us in FP32 and 25.4 in FP64, before 25.0 and 52.4 (rows re-read per sweep in
+// FP64, neighbours clamped); 546 nodes and 110 unknowns (333 x 111 cells) 12.9 and 17.4, before
+// 18.0 and 36.7.  A sweep takes 0.26 us, 0.5 with two nodes a thread, the rows' load 2.3 us (FP32)
+// to 4.8 us (FP64).
 
-size_t tail_lds_bytes(const size_t* nn, int nlev, int bs, size_t elem) {
+size_t tail_level_elems(int nx, int ny, int bs) {
+  const size_t padded = (size_t)(ny + 3) * (nx + 2) + 1, nn = (size_t)(nx + 1) * (ny + 1);
+  return bs * (2 * padded + nn);
+}
+
+size_t tail_lds_bytes(const TailDims* lev, int nlev, int bs, size_t elem) {
   size_t n = 0;
-  for (int l = 0; l + 1 < nlev; ++l) n += 3 * (size_t)bs * nn[l];
-  n += 2 * (size_t)bs * nn[nlev - 1];
+  for (int l = 0; l + 1 < nlev; ++l) n += tail_level_elems(lev[l].nx, lev[l].ny, bs);
+  n += 2 * (size_t)bs * (lev[nlev - 1].nx + 1) * (lev[nlev - 1].ny + 1);
   return n * elem;
 }
 
-// prefetched values of the coarsest inverse per thread (8 threads per row)
-constexpr int kTailDensePre = 8;
-
+// values at one node: the vectors' LDS accesses are one 8- or 16-byte read per node
 template <typename T, int BS>
-struct TailRow {
+struct alignas(sizeof(T) * BS) TailVal {
+  T v[BS];
+};
+
+// the fields of a level that the steps use, read from the argument record once per level
+struct TailGeom {
+  int nx, ny, pitch;  // pitch: nodes per row of the padded vectors
+  unsigned div;
+  template <typename T>
+  __device__ __forceinline__ explicit TailGeom(const TailLevel<T>& L)
+      : nx(L.nx), ny(L.ny), pitch(L.nx + 2), div(L.div) {}
+};
+
+// a thread's node of one level: its coordinates, its place in the padded vectors and its row
+template <typename T, int BS>
+struct TailNode {
   T a[9 * BS * BS];  // a[k*BS*BS + e], k = (dy+1)*3 + (dx+1)
-};
-
-template <typename T, int BS>
-__device__ __forceinline__ void tail_load_row(const TailLevel<T>& L, int v, TailRow<T, BS>& r) {
-  const int nn = (L.nx + 1) * (L.ny + 1);
-  if (v < nn) {
-#pragma unroll
-    for (int e = 0; e < 9 * BS * BS; ++e) r.a[e] = L.st[(size_t)e * nn + v];
+  T inv;             // 1 / det of the 2x2 diagonal block
+  int ix, iy, at;    // at: padded index
+  bool live;
+  __device__ __forceinline__ void place(const TailGeom& g, int v) {
+    iy = (int)(((unsigned)v * g.div) >> 20);  // v / (nx + 1), exact for v, nx + 1 <= 1024
+    ix = v - iy * (g.nx + 1);
+    at = (iy + 1) * g.pitch + ix + 1;
+    live = iy <= g.ny;
   }
-}
-
-// one 9-point operation at node v of a level held in LDS (x, b, y LDS pointers); nb: the
-// node's nine neighbours (clamped into the grid: the stencil entries towards missing
-// neighbours are zero), inv: 1 / det of the 2x2 diagonal block (BS == 2)
-template <typename T, int BS, int OP>
-__device__ __forceinline__ void tail_node(const TailRow<T, BS>& r, const int (&nb)[9], T inv,
-                                          const T* x, const T* b, T* y, T omega, int v) {
-  T acc[BS];
+  // (the diagonal block first: the first sweep needs only that)
+  __device__ __forceinline__ void load(const TailGeom& g, const T* st0, unsigned v) {
+    const unsigned nn = (unsigned)((g.nx + 1) * (g.ny + 1));
+    const auto* st = glob(st0);
+    if (live) {
 #pragma unroll
-  for (int q = 0; q < BS; ++q) acc[q] = T(0);
-  if (OP != kSmoothZero) {
+      for (int o = 0; o < 9; ++o) {
+        const int k = o == 0 ? 4 : o <= 4 ? o - 1 : o;
 #pragma unroll
-    for (int kk = 0; kk < 9; ++kk) {
-      const int j = nb[kk];
-#pragma unroll
-      for (int a = 0; a < BS; ++a)
-#pragma unroll
-        for (int c = 0; c < BS; ++c) acc[a] += r.a[kk * BS * BS + a * BS + c] * x[BS * j + c];
-    }
-  }
-  T res[BS];
-#pragma unroll
-  for (int q = 0; q < BS; ++q) res[q] = b[BS * v + q] - acc[q];
-  if (OP == kResidual) {
-#pragma unroll
-    for (int q = 0; q < BS; ++q) y[BS * v + q] = res[q];
-    return;
-  }
-  T d[BS];
-  if constexpr (BS == 1) {
-    d[0] = res[0] / r.a[4];
-  } else {
-    const T a00 = r.a[16], a01 = r.a[17], a10 = r.a[18], a11 = r.a[19];
-    d[0] = (a11 * res[0] - a01 * res[1]) * inv;
-    d[1] = (a00 * res[1] - a10 * res[0]) * inv;
-  }
-#pragma unroll
-  for (int q = 0; q < BS; ++q) {
-    const T xo = (OP == kSmoothZero) ? T(0) : x[BS * v + q];
-    y[BS * v + q] = xo + omega * d[q];
-  }
-}
-
-// The same operation with the neighbour indices and the diagonal block's inverse determinant
-// formed from the row on the spot (for rows re-read per sweep, where registers are short)
-template <typename T, int BS, int OP>
-__device__ __forceinline__ void tail_node_direct(const TailLevel<T>& L, const TailRow<T, BS>& r,
-                                                 const T* x, const T* b, T* y, T omega, int v) {
-  const int nx = L.nx, ny = L.ny;
-  if (v >= (nx + 1) * (ny + 1)) return;
-  const int ix = v % (nx + 1), iy = v / (nx + 1);
-  T acc[BS];
-#pragma unroll
-  for (int q = 0; q < BS; ++q) acc[q] = T(0);
-  if (OP != kSmoothZero) {
-#pragma unroll
-    for (int kk = 0; kk < 9; ++kk) {
-      const int jx = min(max(ix + kk % 3 - 1, 0), nx), jy = min(max(iy + kk / 3 - 1, 0), ny);
-      const int j = jy * (nx + 1) + jx;
-#pragma unroll
-      for (int a = 0; a < BS; ++a)
-#pragma unroll
-        for (int c = 0; c < BS; ++c) acc[a] += r.a[kk * BS * BS + a * BS + c] * x[BS * j + c];
-    }
-  }
-  T res[BS];
-#pragma unroll
-  for (int q = 0; q < BS; ++q) res[q] = b[BS * v + q] - acc[q];
-  if (OP == kResidual) {
-#pragma unroll
-    for (int q = 0; q < BS; ++q) y[BS * v + q] = res[q];
-    return;
-  }
-  T d[BS];
-  if constexpr (BS == 1) {
-    d[0] = res[0] / r.a[4];
-  } else {
-    const T a00 = r.a[16], a01 = r.a[17], a10 = r.a[18], a11 = r.a[19];
-    const T inv = T(1) / (a00 * a11 - a01 * a10);
-    d[0] = (a11 * res[0] - a01 * res[1]) * inv;
-    d[1] = (a00 * res[1] - a10 * res[0]) * inv;
-  }
-#pragma unroll
-  for (int q = 0; q < BS; ++q) {
-    const T xo = (OP == kSmoothZero) ? T(0) : x[BS * v + q];
-    y[BS * v + q] = xo + omega * d[q];
-  }
-}
-
-// A node's stencil row stays in registers across a level's sweeps when it is small enough
-// (36 floats, 9 doubles) or the workgroup is at most 256 threads; otherwise (the FP64 2x2-block
-// row, 36 doubles, at 1024 threads) it is re-read from global memory (an L2 hit) for each
-// sweep, which keeps the kernel within 128 VGPRs without spills.  (A 256-thread tail with the
-// 47x16 level moved to the band kernels measured slower at N=1000.)  The node's neighbour
-// indices and its diagonal block's inverse determinant are formed once per level.
-template <typename T, int BS>
-struct TailRowHolder {
-  static constexpr bool kKeep = sizeof(T) * 9 * BS * BS <= 144 || kTailThreads <= 256;
-  TailRow<T, BS> row;
-  int nb[9];  // (kKeep only)
-  T inv = T(0);
-  bool live = false;
-  __device__ __forceinline__ static void neighbours(int ix, int iy, int nx, int ny,
-                                                    int (&nb)[9]) {
-#pragma unroll
-    for (int kk = 0; kk < 9; ++kk) {
-      const int jx = min(max(ix + kk % 3 - 1, 0), nx), jy = min(max(iy + kk / 3 - 1, 0), ny);
-      nb[kk] = jy * (nx + 1) + jx;
-    }
-  }
-  __device__ __forceinline__ void level(const TailLevel<T>& L, int v) {
-    if constexpr (kKeep) {
-      const int nx = L.nx, ny = L.ny;
-      live = v < (nx + 1) * (ny + 1);
-      if (!live) return;
-      neighbours(v % (nx + 1), v / (nx + 1), nx, ny, nb);
-      tail_load_row<T, BS>(L, v, row);
-    }
-  }
-  // the diagonal block's inverse determinant, formed at the level's first sweep (after the
-  // phase that the row loads overlap)
-  __device__ __forceinline__ void finish() {
-    if constexpr (kKeep && BS == 2)
-      if (live) inv = diag_inv(row);
-  }
-  __device__ __forceinline__ static T diag_inv(const TailRow<T, BS>& r) {
-    return T(1) / (r.a[16] * r.a[19] - r.a[17] * r.a[18]);
-  }
-  template <int OP>
-  __device__ __forceinline__ void sweep(const TailLevel<T>& L, const T* x, const T* b, T* y,
-                                        T omega, int v) {
-    if constexpr (kKeep) {
-      if (live) tail_node<T, BS, OP>(row, nb, inv, x, b, y, omega, v);
-    } else {
-      tail_load_row<T, BS>(L, v, row);
-      tail_node_direct<T, BS, OP>(L, row, x, b, y, omega, v);
-    }
-  }
-};
-
-template <typename T, int BS>
-__device__ __forceinline__ void tail_vcycle_body(const BlkId blk, const TailDesc<T>& d) {
-  extern __shared__ __align__(16) unsigned char tail_lds[];
-  T* lds = reinterpret_cast<T*>(tail_lds);
-  const int tid = threadIdx.x;
-  const int nl = d.nlev;  // levels 0..nl-2 are 9-point, level nl-1 is the dense coarsest
-  // ping-pong parity: the first sweep writes buffer (S-1)%2 so that after S sweeps the
-  // iterate is in buffer 0; after the pre-sweeps it is in buffer nu_post%2 on every level
-  const int w_first = (d.nu_pre + d.nu_post - 1) & 1;
-  const int w_mid = d.nu_post & 1;
-  // this thread's part of its row of the coarsest inverse, loaded now so that its latency
-  // passes during the down leg (systems of at most 8 kPre unknowns; FP32 only: the FP64
-  // kernel has no registers to spare)
-  constexpr int kPre = sizeof(T) == 4 ? kTailDensePre : 1;
-  double dpre[kPre];
-  {
-    const int row = tid >> 3, part = tid & 7, n = d.cn;
-#pragma unroll
-    for (int k = 0; k < kPre; ++k)
-      dpre[k] = (sizeof(T) == 4 && n <= 8 * kPre && row < n && part + 8 * k < n)
-                    ? d.dense[(size_t)row * n + part + 8 * k]
-                    : 0.0;
-  }
-  // The holder keeps one level's rows.  Each level's rows are requested one phase before
-  // their first sweep (before the right-hand side's load, the restriction or the
-  // prolongation), so their load latency passes during that phase; the deepest 9-point
-  // level's rows serve both legs.
-  TailRowHolder<T, BS> rh;
-  rh.level(d.lev[0], tid);
-  {  // top-level right-hand side into LDS
-    const TailLevel<T>& L = d.lev[0];
-    const int n = BS * (L.nx + 1) * (L.ny + 1);
-    T* b = lds + L.off + 2 * n;
-    for (int i = tid; i < n; i += kTailThreads) b[i] = d.b_in[i];
-  }
-  __syncthreads();
-  for (int l = 0; l + 1 < nl; ++l) {
-    const TailLevel<T>& L = d.lev[l];
-    const int nn = (L.nx + 1) * (L.ny + 1);
-    T* const b0 = lds + L.off;
-    T* const b1 = b0 + BS * nn;
-    const T* b = b0 + 2 * BS * nn;
-    int w = w_first;
-    rh.finish();
-    rh.template sweep<kSmoothZero>(L, nullptr, b, w ? b1 : b0, d.omega[0], tid);
-    __syncthreads();
-    for (int k = 1; k < d.nu_pre; ++k) {
-      rh.template sweep<kSmooth>(L, w ? b1 : b0, b, w ? b0 : b1, d.omega[k], tid);
-      __syncthreads();
-      w ^= 1;
-    }
-    T* const spare = w ? b0 : b1;  // the residual goes to the free ping-pong buffer
-    rh.template sweep<kResidual>(L, w ? b1 : b0, b, spare, T(0), tid);
-    if (l + 2 < nl) rh.level(d.lev[l + 1], tid);  // (the dense coarsest has no rows)
-    __syncthreads();
-    const TailLevel<T>& C = d.lev[l + 1];
-    const int nnc = (C.nx + 1) * (C.ny + 1);
-    T* cb = lds + C.off + (l + 2 == nl ? 0 : 2 * BS * nnc);
-    if (tid < nnc) restrict_bilinear_node<T, BS>(L.nx, L.ny, C.nx, C.ny, d.fixed, spare, cb, tid);
-    __syncthreads();
-  }
-  {  // dense coarsest: x = Ainv b, 8 lanes per row (cn <= 128 rows)
-    const TailLevel<T>& C = d.lev[nl - 1];
-    const int n = d.cn;
-    const T* cb = lds + C.off;
-    T* cx = lds + C.off + n;
-    const int part = tid & 7;
-    for (int row0 = 0; row0 < n; row0 += kTailThreads / 8) {  // (all lanes loop alike)
-      const int row = row0 + (tid >> 3);
-      double s = 0.0;
-      if (row < n) {
-        if (sizeof(T) == 4 && n <= 8 * kPre && row0 == 0) {  // the row was loaded at the start
-#pragma unroll
-          for (int k = 0; k < kPre; ++k)
-            if (part + 8 * k < n) s += dpre[k] * (double)cb[part + 8 * k];
-        } else {
-          const double* arow = d.dense + (size_t)row * n;
-          for (int j = part; j < n; j += 8) s += arow[j] * (double)cb[j];
+        for (int e = 0; e < BS * BS; ++e) {
+          const auto* se = st + (size_t)((k * BS * BS + e) * nn);  // (uniform)
+          a[k * BS * BS + e] = se[v];
         }
       }
-      s += __shfl_down(s, 4, 8);
-      s += __shfl_down(s, 2, 8);
-      s += __shfl_down(s, 1, 8);
-      if (row < n && part == 0) cx[row] = (T)s;
+    }
+  }
+  __device__ __forceinline__ void finish() {
+    if constexpr (BS == 2)
+      if (live) inv = T(1) / (a[16] * a[19] - a[17] * a[18]);
+  }
+  __device__ __forceinline__ TailVal<T, BS> solve_diag(const TailVal<T, BS>& r) const {
+    TailVal<T, BS> d;
+    if constexpr (BS == 1) {
+      d.v[0] = r.v[0] / a[4];
+    } else {
+      d.v[0] = (a[19] * r.v[0] - a[17] * r.v[1]) * inv;
+      d.v[1] = (a[16] * r.v[1] - a[18] * r.v[0]) * inv;
+    }
+    return d;
+  }
+  // b - A x at the node (one chain of sums per row of neighbours), xc = x there
+  __device__ __forceinline__ TailVal<T, BS> residual(int pitch, const TailVal<T, BS>* x,
+                                                     const TailVal<T, BS>& b,
+                                                     TailVal<T, BS>& xc) const {
+    T acc[3][BS];
+#pragma unroll
+    for (int dy = 0; dy < 3; ++dy) {
+      const TailVal<T, BS>* row = x + at + (dy - 1) * pitch;
+      const TailVal<T, BS> u[3] = {row[-1], row[0], row[1]};
+      if (dy == 1) xc = u[1];
+#pragma unroll
+      for (int p = 0; p < BS; ++p) {
+        acc[dy][p] = T(0);
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+          for (int c = 0; c < BS; ++c)
+            acc[dy][p] += a[(dy * 3 + dx) * BS * BS + p * BS + c] * u[dx].v[c];
+      }
+    }
+    TailVal<T, BS> r;
+#pragma unroll
+    for (int q = 0; q < BS; ++q) r.v[q] = b.v[q] - ((acc[0][q] + acc[1][q]) + acc[2][q]);
+    return r;
+  }
+  __device__ __forceinline__ void smooth(int pitch, const TailVal<T, BS>* x,
+                                         const TailVal<T, BS>* b, TailVal<T, BS>* y, T omega,
+                                         int v) const {
+    if (!live) return;
+    TailVal<T, BS> xc;
+    const TailVal<T, BS> d = solve_diag(residual(pitch, x, b[v], xc));
+#pragma unroll
+    for (int q = 0; q < BS; ++q) xc.v[q] += omega * d.v[q];
+    y[at] = xc;
+  }
+};
+
+// The bilinear transfers between two levels (coarse cells = ceil(fine / 2) per axis): an even
+// fine node lies on coarse node f / 2, the last node of an odd count on the last coarse node,
+// any other odd node half way.  Restriction at coarse node I: its fine node p = min(2I, nf) and
+// the halves from p - 1 and p + 1 that lie half way (the border is zero).  Products with 0, 1/2
+// and 1 are exact; the sum is kept in double, as in the launch-per-step transfers.
+template <typename T, int BS>
+__device__ __forceinline__ TailVal<T, BS> tail_restrict(const TailGeom& f, const TailVal<T, BS>* rf,
+                                                        int I, int J, bool fixed) {
+  const int px = min(2 * I, f.nx), py = min(2 * J, f.ny);
+  const double wx[3] = {(px & 1) ? 0.0 : 0.5, 1.0, ((px & 1) || px + 1 == f.nx) ? 0.0 : 0.5};
+  const double wy[3] = {(py & 1) ? 0.0 : 0.5, 1.0, ((py & 1) || py + 1 == f.ny) ? 0.0 : 0.5};
+  const TailVal<T, BS>* c = rf + (py + 1) * f.pitch + px + 1;
+  double acc[BS];
+#pragma unroll
+  for (int q = 0; q < BS; ++q) acc[q] = 0.0;
+#pragma unroll
+  for (int dy = 0; dy < 3; ++dy) {
+    const TailVal<T, BS> u[3] = {c[(dy - 1) * f.pitch - 1], c[(dy - 1) * f.pitch],
+                                 c[(dy - 1) * f.pitch + 1]};
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+      for (int q = 0; q < BS; ++q) acc[q] += wy[dy] * wx[dx] * (double)u[dx].v[q];
+  }
+  TailVal<T, BS> b;
+#pragma unroll
+  for (int q = 0; q < BS; ++q) b.v[q] = fixed ? T(0) : (T)acc[q];
+  return b;
+}
+
+// xf += P ec at the fine node (ix, iy); ec: coarse node (0, 0), rows of cp nodes
+template <typename T, int BS>
+__device__ __forceinline__ void tail_prolong(const TailGeom& f, int ix, int iy,
+                                             const TailVal<T, BS>* ec, int cp,
+                                             TailVal<T, BS>& xf) {
+  const T x1 = (ix & 1) ? (ix == f.nx ? T(1) : T(0.5)) : T(0), x0 = T(1) - x1;
+  const T y1 = (iy & 1) ? (iy == f.ny ? T(1) : T(0.5)) : T(0), y0 = T(1) - y1;
+  // (an even node's second neighbour has weight zero and may not exist: its own is read)
+  const int ox = (ix & 1) ? 1 : 0, oy = (iy & 1) ? cp : 0;
+  const TailVal<T, BS>* e = ec + (iy >> 1) * cp + (ix >> 1);
+  const TailVal<T, BS> e00 = e[0], e10 = e[ox], e01 = e[oy], e11 = e[oy + ox];
+  TailVal<T, BS> x = xf;
+#pragma unroll
+  for (int q = 0; q < BS; ++q)
+    x.v[q] += x0 * y0 * e00.v[q] + x1 * y0 * e10.v[q] + x0 * y1 * e01.v[q] + x1 * y1 * e11.v[q];
+  xf = x;
+}
+
+// Workgroups are dealt to the 8 XCDs in turn, so blocks 8, 16, .. share block 0's L2, which holds
+// nothing of earlier launches: they read the rows and the coarsest inverse once (a value per 64
+// bytes), so that block 0, whose own misses are limited, finds them there.
+template <typename T, int BS>
+__device__ __forceinline__ void tail_fetch(const TailDesc<T>& d, int part, int parts) {
+  auto fetch = [&](const void* p, int bytes) {
+    const auto* q = glob(static_cast<const unsigned char*>(p));
+    for (int i = 64 * ((int)threadIdx.x + part * kTailWg); i < bytes; i += 64 * kTailWg * parts) {
+      const int x = q[i];
+      asm volatile("" ::"v"(x));  // (the value is not used)
+    }
+  };
+  for (int l = 0; l + 1 < d.nlev; ++l)
+    fetch(d.lev[l].st,
+          9 * BS * BS * (int)sizeof(T) * (d.lev[l].nx + 1) * (d.lev[l].ny + 1));
+  fetch(d.dense, d.cn * d.cn * (int)sizeof(double));
+}
+
+// The workgroup has kTailWg threads.  The top level has up to two nodes per thread, the levels
+// below it one (find_tail sees to that), and each thread keeps its top-level rows from the down
+// leg to the up leg: one CU reads 64 bytes per clock, so reading the rows of 816 nodes again
+// would take 1 us (FP32) or 2 us (FP64).  Where three rows do not fit the 256 registers (FP64
+// 2x2 blocks: 72 each), the levels below use the second node's, which is read again.
+template <typename T, int BS>
+__device__ __forceinline__ void tail_vcycle_body(const BlkId blk, const TailDesc<T>& d) {
+  using V = TailVal<T, BS>;
+  using Node = TailNode<T, BS>;
+  if (blk.id != 0) {
+    if (blk.id % 8 == 0) tail_fetch<T, BS>(d, blk.id / 8 - 1, kTailHelpers);
+    return;
+  }
+  extern __shared__ __align__(16) unsigned char tail_lds[];
+  T* const lds = reinterpret_cast<T*>(tail_lds);
+  const int tid = threadIdx.x;
+  const int nl = d.nlev;  // levels 0..nl-2 have rows, level nl-1 is the dense coarsest
+  const int nu_pre = d.nu_pre, nu_post = d.nu_post;
+  const unsigned fixed = d.fixed;
+  // (selects on scalars: no load between two barriers)
+  const T om0 = d.omega[0], om1 = d.omega[1], om2 = d.omega[2], om3 = d.omega[3];
+  const T om4 = d.omega[4], om5 = d.omega[5], om6 = d.omega[6], om7 = d.omega[7];
+  static_assert(kMaxNu == 8, "one step size per sweep");
+  auto omega = [=](int j) {
+    return j < 4 ? (j < 2 ? (j ? om1 : om0) : (j == 2 ? om2 : om3))
+                 : (j < 6 ? (j == 4 ? om4 : om5) : (j == 6 ? om6 : om7));
+  };
+  // ping-pong parity: the first sweep writes buffer (S-1)%2 so that after S sweeps the
+  // iterate is in buffer 0; after the pre-sweeps it is in buffer nu_post%2 on every level
+  const int w_first = (nu_pre + nu_post - 1) & 1;
+  const int w_mid = nu_post & 1;
+  constexpr bool kKeep = sizeof(T) * BS * BS <= 16;
+  Node top[kKeep ? 3 : 2];
+  V rt[kKeep ? 3 : 2];
+  Node* const low = top + (kKeep ? 2 : 1);
+  V* const rl = rt + (kKeep ? 2 : 1);
+  const TailGeom g0(d.lev[0]);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int v = tid + k * kTailWg;
+    top[k].place(g0, v);
+    top[k].load(g0, d.lev[0].st, v);
+#pragma unroll
+    for (int q = 0; q < BS; ++q) rt[k].v[q] = top[k].live ? glob(d.b_in)[BS * v + q] : T(0);
+  }
+  {  // borders (and all vectors) to zero, in 16-byte pieces
+    float4* z = reinterpret_cast<float4*>(tail_lds);
+    const int n16 = (d.zero * (int)sizeof(T) + 15) / 16;
+    for (int i = tid; i < n16; i += kTailWg) z[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  // the coarsest inverse goes to LDS behind the vectors, its latency passing with the rows'
+  double* const dl = reinterpret_cast<double*>(tail_lds + d.dense_off);
+  if (d.dense_off)
+    for (int i = tid; i < d.cn * d.cn; i += kTailWg) dl[i] = glob(d.dense)[i];
+  __syncthreads();
+  // down leg of one level with its nodes (one per thread, or two), from the right-hand side in
+  // the thread's registers to the residual in `spare`
+  auto down = [&](auto per, Node* nodes, const V* rhs, const TailGeom& g, int off,
+                  int padded) -> V* {
+    constexpr int kPer = decltype(per)::value;
+    V* const b0 = reinterpret_cast<V*>(lds + off);
+    V* const b1 = reinterpret_cast<V*>(lds + off + padded);
+    V* const b = reinterpret_cast<V*>(lds + off + 2 * padded);
+    int w = w_first;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      nodes[k].finish();
+      if (nodes[k].live) {  // the first sweep from zero needs only the node itself
+        V s = nodes[k].solve_diag(rhs[k]);
+#pragma unroll
+        for (int q = 0; q < BS; ++q) s.v[q] *= om0;
+        b[tid + k * kTailWg] = rhs[k];
+        (w ? b1 : b0)[nodes[k].at] = s;
+      }
     }
     __syncthreads();
-  }
-  for (int l = nl - 2; l >= 0; --l) {
-    const TailLevel<T>& L = d.lev[l];
-    const TailLevel<T>& C = d.lev[l + 1];
-    const int nn = (L.nx + 1) * (L.ny + 1);
-    T* const b0 = lds + L.off;
-    T* const b1 = b0 + BS * nn;
-    const T* b = b0 + 2 * BS * nn;
-    const T* cx = lds + C.off + (l + 2 == nl ? d.cn : 0);
-    int w = w_mid;
-    if (tid < nn) prolong_bilinear_node<T, BS>(L.nx, L.ny, C.nx, C.ny, d.fixed, cx, w ? b1 : b0, tid);
-    if (d.nu_post == 0 && l > 0) rh.level(d.lev[l - 1], tid);
-    __syncthreads();
-    if (l + 2 < nl) rh.finish();  // (the deepest level's is still set from the down leg)
-    for (int k = 0; k < d.nu_post; ++k) {
-      rh.template sweep<kSmooth>(L, w ? b1 : b0, b, w ? b0 : b1, d.omega[k], tid);
-      if (k + 1 == d.nu_post && l > 0) rh.level(d.lev[l - 1], tid);
+    for (int j = 1; j < nu_pre; ++j) {
+      const T o = omega(j);
+#pragma unroll
+      for (int k = 0; k < kPer; ++k)
+        nodes[k].smooth(g.pitch, w ? b1 : b0, b, w ? b0 : b1, o, tid + k * kTailWg);
       __syncthreads();
       w ^= 1;
     }
-    if (l == 0) {
-      const int n = BS * nn;
-      for (int i = tid; i < n; i += kTailThreads) d.x_out[i] = b0[i];
+    V* const spare = w ? b0 : b1;  // the residual goes to the free ping-pong buffer
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+      if (nodes[k].live) {
+        V xc;
+        spare[nodes[k].at] =
+            nodes[k].residual(g.pitch, w ? b1 : b0, b[tid + k * kTailWg], xc);
+      }
+    return spare;
+  };
+  // up leg: prolongation from the level below (ec, rows of cp nodes) and the post-sweeps; the
+  // result is in buffer 0
+  auto up = [&](auto per, Node* nodes, const TailGeom& g, int off, int padded, const V* ec,
+                int cp) {
+    constexpr int kPer = decltype(per)::value;
+    V* const b0 = reinterpret_cast<V*>(lds + off);
+    V* const b1 = reinterpret_cast<V*>(lds + off + padded);
+    const V* b = reinterpret_cast<const V*>(lds + off + 2 * padded);
+    int w = w_mid;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+      if (nodes[k].live && !node_fixed(fixed, nodes[k].ix, nodes[k].iy, g.nx, g.ny))
+        tail_prolong<T, BS>(g, nodes[k].ix, nodes[k].iy, ec, cp, (w ? b1 : b0)[nodes[k].at]);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) nodes[k].finish();  // (rows requested before the call)
+    for (int j = 0; j < nu_post; ++j) {
+      const T o = omega(j);
+#pragma unroll
+      for (int k = 0; k < kPer; ++k)
+        nodes[k].smooth(g.pitch, w ? b1 : b0, b, w ? b0 : b1, o, tid + k * kTailWg);
+      __syncthreads();
+      w ^= 1;
     }
+  };
+  const V* spare = nullptr;
+  for (int l = 0; l + 1 < nl; ++l) {
+    const TailGeom g(d.lev[l]), c(d.lev[l + 1]);
+    const int off = d.lev[l].off, padded = d.lev[l].padded, coff = d.lev[l + 1].off;
+    const bool rows = l + 2 < nl;  // (the dense coarsest has none)
+    const T* cst = d.lev[l + 1].st;
+    spare = l == 0 ? down(std::integral_constant<int, 2>(), top, rt, g, off, padded)
+                   : down(std::integral_constant<int, 1>(), low, rl, g, off, padded);
+    // the next level's rows are requested before its right-hand side is formed (the deepest
+    // ones then serve both legs)
+    if (rows) {
+      low[0].place(c, tid);
+      low[0].load(c, cst, tid);
+      __syncthreads();
+      if (low[0].live)
+        rl[0] = tail_restrict<T, BS>(g, spare, low[0].ix, low[0].iy,
+                                     node_fixed(fixed, low[0].ix, low[0].iy, c.nx, c.ny));
+    } else {
+      __syncthreads();
+      const int J = (int)(((unsigned)tid * c.div) >> 20), I = tid - J * (c.nx + 1);
+      if (J <= c.ny)  // (at most 128 nodes)
+        reinterpret_cast<V*>(lds + coff)[tid] =
+            tail_restrict<T, BS>(g, spare, I, J, node_fixed(fixed, I, J, c.nx, c.ny));
+      __syncthreads();
+    }
+  }
+  const TailGeom gc(d.lev[nl - 1]);
+  const int coff = d.lev[nl - 1].off;
+  {  // dense coarsest: x = Ainv b, 4 lanes per row (cn <= 128 rows)
+    const int n = d.cn;
+    const T* cb = lds + coff;
+    T* cx = lds + coff + n;
+    const int part = tid & 3, row = tid >> 2;
+    double s0 = 0.0, s1 = 0.0;
+    if (row < n) {
+      if (d.dense_off) {
+        const double* arow = dl + row * n;
+        int j = part;
+        for (; j + 4 < n; j += 8) {
+          s0 += arow[j] * (double)cb[j];
+          s1 += arow[j + 4] * (double)cb[j + 4];
+        }
+        if (j < n) s0 += arow[j] * (double)cb[j];
+      } else {
+        const auto* arow = glob(d.dense) + (size_t)row * n;
+#pragma unroll 8
+        for (int j = part; j < n; j += 4) s0 += arow[j] * (double)cb[j];
+      }
+    }
+    s0 += s1;
+    s0 += __shfl_down(s0, 2, 4);
+    s0 += __shfl_down(s0, 1, 4);
+    if (row < n && part == 0) cx[row] = (T)s0;
+    __syncthreads();
+  }
+  for (int l = nl - 2; l >= 1; --l) {
+    const TailGeom g(d.lev[l]);
+    const bool dense = l + 2 == nl;
+    const int cp = dense ? gc.nx + 1 : d.lev[l + 1].nx + 2;
+    const V* ec = dense ? reinterpret_cast<const V*>(lds + coff + d.cn)
+                        : reinterpret_cast<const V*>(lds + d.lev[l + 1].off) + cp + 1;
+    if (!dense) {  // (the deepest level's rows are there from the down leg)
+      low[0].place(g, tid);
+      low[0].load(g, d.lev[l].st, tid);
+    }
+    up(std::integral_constant<int, 1>(), low, g, d.lev[l].off, d.lev[l].padded, ec, cp);
+  }
+  {
+    if (!kKeep && nl > 2) {
+      top[1].place(g0, tid + kTailWg);
+      top[1].load(g0, d.lev[0].st, tid + kTailWg);
+    }
+    const bool dense = nl == 2;
+    const int cp = dense ? gc.nx + 1 : d.lev[1].nx + 2;
+    const V* ec = dense ? reinterpret_cast<const V*>(lds + coff + d.cn)
+                        : reinterpret_cast<const V*>(lds + d.lev[1].off) + cp + 1;
+    up(std::integral_constant<int, 2>(), top, g0, d.lev[0].off, d.lev[0].padded, ec, cp);
+    const V* b0 = reinterpret_cast<const V*>(lds + d.lev[0].off);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (top[k].live) {
+        const V x = b0[top[k].at];
+#pragma unroll
+        for (int q = 0; q < BS; ++q) glob(d.x_out)[BS * (tid + k * kTailWg) + q] = x.v[q];
+      }
   }
 }
 
 template <typename T, int BS>
-__global__ __launch_bounds__(kTailThreads) void k_tail_vcycle(TailDesc<T> d) {
+__global__ __launch_bounds__(kTailWg) void k_tail_vcycle(TailDesc<T> d) {
   tail_vcycle_body<T, BS>(hw_blk(), d);
 }
 
 template <typename T, int BS>
-hipError_t tail_vcycle(const TailDesc<T>& d, size_t lds_bytes, hipStream_t s) {
-  if (d.nlev < 2 || d.nlev > kMaxTail || d.cn > 128 || lds_bytes > kTailLdsBytes ||
-      d.nu_pre < 1 || d.nu_pre > kMaxNu || d.nu_post < 0 || d.nu_post > kMaxNu)
+hipError_t tail_vcycle(const TailDesc<T>& d0, hipStream_t s) {
+  TailDesc<T> d = d0;
+  if (d.nlev < 2 || d.nlev > kMaxTail || d.cn > 128 || d.nu_pre < 1 || d.nu_pre > kMaxNu ||
+      d.nu_post < 0 || d.nu_post > kMaxNu)
     return hipErrorInvalidValue;
-  for (int l = 0; l + 1 < d.nlev; ++l)
-    if ((d.lev[l].nx + 1) * (d.lev[l].ny + 1) > kTailThreads) return hipErrorInvalidValue;
-  TMX_LAUNCH_OR_RECORD(kTailThreads, (tail_vcycle_body<T, BS>), 1, lds_bytes, s, (k_tail_vcycle<T, BS>), d);
+  TailDims dims[kMaxTail];
+  int off = 0;
+  for (int l = 0; l < d.nlev; ++l) {
+    TailLevel<T>& L = d.lev[l];
+    const int nn = (L.nx + 1) * (L.ny + 1);
+    // one node per thread, two on the top level
+    if (L.nx < 1 || L.ny < 1 || nn > (l == 0 ? 2 : 1) * kTailWg) return hipErrorInvalidValue;
+    dims[l] = TailDims{L.nx, L.ny};
+    L.div = (unsigned)(((1u << 20) + L.nx) / (L.nx + 1));  // ceil(2^20 / (nx + 1))
+    L.padded = BS * ((L.ny + 3) * (L.nx + 2) + 1);
+    L.off = off;
+    off += l + 1 < d.nlev ? (int)tail_level_elems(L.nx, L.ny, BS) : 2 * BS * nn;
+  }
+  if (BS * (d.lev[d.nlev - 1].nx + 1) * (d.lev[d.nlev - 1].ny + 1) != d.cn)
+    return hipErrorInvalidValue;
+  d.zero = d.lev[d.nlev - 1].off;
+  size_t lds = tail_lds_bytes(dims, d.nlev, BS, sizeof(T));
+  if (lds > kTailLdsBytes) return hipErrorInvalidValue;
+  lds = (lds + 15) & ~size_t(15);  // (the clearing writes whole 16-byte pieces)
+  d.dense_off = 0;
+  const size_t need = sizeof(double) * d.cn * d.cn;
+  if (d.cn <= 64 && lds + need <= kTailLdsMax) {
+    d.dense_off = (int)lds;
+    lds += need;
+  }
+  if (lds > 64 * 1024 && !active_recorder()) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tail_vcycle<T, BS>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  TMX_LAUNCH_OR_RECORD(kTailWg, (tail_vcycle_body<T, BS>), 1 + 8 * kTailHelpers, lds, s,
+                       (k_tail_vcycle<T, BS>), d);
   return hipGetLastError();
 }
-template hipError_t tail_vcycle<double, 1>(const TailDesc<double>&, size_t, hipStream_t);
-template hipError_t tail_vcycle<double, 2>(const TailDesc<double>&, size_t, hipStream_t);
-template hipError_t tail_vcycle<float, 1>(const TailDesc<float>&, size_t, hipStream_t);
-template hipError_t tail_vcycle<float, 2>(const TailDesc<float>&, size_t, hipStream_t);
+template hipError_t tail_vcycle<double, 1>(const TailDesc<double>&, hipStream_t);
+template hipError_t tail_vcycle<double, 2>(const TailDesc<double>&, hipStream_t);
+template hipError_t tail_vcycle<float, 1>(const TailDesc<float>&, hipStream_t);
+template hipError_t tail_vcycle<float, 2>(const TailDesc<float>&, hipStream_t);
 
 // Galerkin product R A P for tensor-product linear (bilinear) coarsening, one thread per
 // coarse node (I, J) and coarse stencil direction kc (nine threads per node): the thread forms

@@ -153,13 +153,15 @@ void Hierarchy::find_tail() {
   const int lastl = (int)levels_.size() - 1;
   tail_ = -1;
   if (lastl >= 1 && bs_ * levels_[lastl].nn <= 128) {
-    const size_t cap = (size_t)std::min(tail_nodes_, kTailThreads);
+    const size_t cap = (size_t)std::min(tail_nodes_, kTailNodes);
     int t = lastl;
     while (t - 1 >= 1 && lastl - (t - 1) + 1 <= kMaxTail && levels_[t - 1].kind == kStencil &&
-           levels_[t - 1].nn <= cap && !levels_[t].nested_from_prev) {
-      size_t nn[kMaxTail];
-      for (int l = t - 1; l <= lastl; ++l) nn[l - (t - 1)] = levels_[l].nn;
-      if (tail_lds_bytes(nn, lastl - (t - 1) + 1, bs_, sizeof(double)) > kTailLdsBytes) break;
+           levels_[t - 1].nn <= cap && levels_[t].nn <= (size_t)kTailWg &&
+           !levels_[t].nested_from_prev) {
+      TailDims dims[kMaxTail];
+      for (int l = t - 1; l <= lastl; ++l)
+        dims[l - (t - 1)] = TailDims{levels_[l].nx, levels_[l].ny};
+      if (tail_lds_bytes(dims, lastl - (t - 1) + 1, bs_, sizeof(double)) > kTailLdsBytes) break;
       --t;
     }
     tail_ = t;
@@ -628,21 +630,15 @@ static int tail_launch(Hierarchy& h, const T* b, T* x, hipStream_t s) {
   d.dense = h.dense_.get();
   d.b_in = b;
   d.x_out = x;
-  size_t nn[kMaxTail];
-  int off = 0;
   for (int l = h.tail_; l <= last; ++l) {
     Level& L = h.levels_[l];
     TailLevel<T>& t = d.lev[l - h.tail_];
     t.nx = L.nx;
     t.ny = L.ny;
     t.st = PrecBufs<T>::st(L);
-    t.off = off;
-    off += (l < last ? 3 : 2) * h.bs_ * (int)L.nn;
-    nn[l - h.tail_] = L.nn;
   }
-  const size_t lds = tail_lds_bytes(nn, d.nlev, h.bs_, sizeof(T));
-  if (h.bs_ == 2) TMX_HIP((tail_vcycle<T, 2>(d, lds, s)));
-  else TMX_HIP((tail_vcycle<T, 1>(d, lds, s)));
+  if (h.bs_ == 2) TMX_HIP((tail_vcycle<T, 2>(d, s)));
+  else TMX_HIP((tail_vcycle<T, 1>(d, s)));
   return 0;
 }
 
