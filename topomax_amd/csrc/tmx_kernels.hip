@@ -2936,17 +2936,36 @@ __global__ __launch_bounds__(1024) void k_dense_invert_lds(int n, double* __rest
   dense_invert_lds_body(hw_blk(), n, a);
 }
 
-// The same Gauss-Jordan steps with the matrix in registers, for n <= 4 G: thread (ti, tj) of a
-// G x G arrangement holds the 4 x 4 block of rows 4 ti.. and columns 4 tj..; step k publishes
-// column k and row k through LDS (double-buffered, so one barrier per step) and every thread
-// updates its block from them.  Per step each thread reads 8 values from LDS for its 16
-// updates, a quarter of the LDS traffic of the LDS-resident form, with the same arithmetic.
-// G is the smallest of 8, 16, 32 that covers n: a barrier of fewer waves per step (one wave
-// for n <= 32).
+// The inverse by Gauss-Jordan steps on 4 x 4 blocks with the matrix in registers, for symmetric
+// positive definite matrices of n <= 4 G: thread (ti, tj) of a G x G arrangement holds the block
+// of rows 4 ti.. and columns 4 tj.. (the identity beyond n).  Step k, with the pivot block P:
+// the threads of block row k form and publish R = P^-1 M_k*, those of block column k publish
+// C = M_*k, and every thread updates M -= C R (block column k becomes -C P^-1, block row k R).
+// The steps form one dependent chain, so what counts is their number and what each waits for:
+// a quarter of the scalar steps, two barriers each, and the next pivot's inverse formed by its
+// own thread alone right after its update, so that a step's reciprocals (four, one after the
+// other) are off the other threads' path.  126 unknowns: 71 us (one unknown per step: 154);
+// 72 unknowns: 45 us (91); 42 unknowns: 21 us (42).  G is the smallest of 8, 16, 32 that covers n.
 constexpr int kDenseRegMax = 128;
+__device__ __forceinline__ void invert4(double (&p)[4][4]) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const double rp = 1.0 / p[k][k];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) p[k][j] = j == k ? rp : p[k][j] * rp;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (i == k) continue;
+      const double c = p[i][k];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) p[i][j] = j == k ? -c * rp : p[i][j] - c * p[k][j];
+    }
+  }
+}
+
 template <int G>
 __device__ __forceinline__ void dense_invert_reg_body(const BlkId, int n, double* a) {
-  __shared__ double colb[2][4 * G], rowb[2][4 * G];
+  __shared__ double pinv[16], row[16][G], col[G][16];
   const int tid = (int)threadIdx.x, ti = tid / G, tj = tid % G;
   const int i0 = 4 * ti, j0 = 4 * tj;
   double m[4][4];
@@ -2954,47 +2973,77 @@ __device__ __forceinline__ void dense_invert_reg_body(const BlkId, int n, double
   for (int r = 0; r < 4; ++r)
 #pragma unroll
     for (int c = 0; c < 4; ++c)
-      m[r][c] = (i0 + r < n && j0 + c < n) ? a[(size_t)(i0 + r) * n + j0 + c] : 0.0;
-  for (int k = 0; k < n; ++k) {
-    const int buf = k & 1;
-    if (tj == (k >> 2)) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if ((k & 3) == 0) colb[buf][i0 + r] = m[r][0];
-        else if ((k & 3) == 1) colb[buf][i0 + r] = m[r][1];
-        else if ((k & 3) == 2) colb[buf][i0 + r] = m[r][2];
-        else colb[buf][i0 + r] = m[r][3];
-    }
-    if (ti == (k >> 2)) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        if ((k & 3) == 0) rowb[buf][j0 + c] = m[0][c];
-        else if ((k & 3) == 1) rowb[buf][j0 + c] = m[1][c];
-        else if ((k & 3) == 2) rowb[buf][j0 + c] = m[2][c];
-        else rowb[buf][j0 + c] = m[3][c];
-    }
-    __syncthreads();
-    const double rp = 1.0 / colb[buf][k];
-    double cl[4], rw[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) cl[r] = colb[buf][i0 + r];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) rw[c] = rowb[buf][j0 + c];
+      m[r][c] = (i0 + r < n && j0 + c < n) ? glob(a)[(size_t)(i0 + r) * n + j0 + c]
+                                           : (i0 + r == j0 + c ? 1.0 : 0.0);
+  auto publish_pivot = [&]() {
+    double p[4][4];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int i = i0 + r, j = j0 + c;
-        const double mkj = (j == k) ? rp : rw[c] * rp;  // the scaled pivot row
-        if (i == k) m[r][c] = mkj;
-        else m[r][c] = (j == k) ? -cl[r] * rp : m[r][c] - cl[r] * mkj;
+      for (int c = 0; c < 4; ++c) p[r][c] = m[r][c];
+    invert4(p);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) pinv[4 * r + c] = p[r][c];
+  };
+  if (tid == 0) publish_pivot();
+  const int steps = (n + 3) / 4;
+  for (int k = 0; k < steps; ++k) {
+    __syncthreads();  // the pivot's inverse is there; the last step's R and C are read
+    if (ti == k) {
+      double p[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) p[e] = pinv[e];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          double x = p[4 * r] * m[0][c];
+#pragma unroll
+          for (int q = 1; q < 4; ++q) x += p[4 * r + q] * m[q][c];
+          row[4 * r + c][tj] = tj == k ? p[4 * r + c] : x;
+        }
+    }
+    if (tj == k) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) col[ti][4 * r + c] = m[r][c];
+    }
+    __syncthreads();
+    double rr[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) rr[q][c] = row[4 * q + c][tj];
+    if (ti == k) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) m[r][c] = rr[r][c];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        double cl[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) cl[q] = col[ti][4 * r + q];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          double x = tj == k ? 0.0 : m[r][c];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) x -= cl[q] * rr[q][c];
+          m[r][c] = x;
+        }
       }
+      if (ti == k + 1 && tj == k + 1) publish_pivot();
+    }
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
     for (int c = 0; c < 4; ++c)
-      if (i0 + r < n && j0 + c < n) a[(size_t)(i0 + r) * n + j0 + c] = m[r][c];
+      if (i0 + r < n && j0 + c < n) glob(a)[(size_t)(i0 + r) * n + j0 + c] = m[r][c];
 }
 
 template <int G>
