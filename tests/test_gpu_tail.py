@@ -51,3 +51,24 @@ def test_tail_equals_launch_per_step(nx, ny, sweeps):
         for a, b in zip(*out):
             assert torch.isfinite(b).all()
             assert float((a - b).norm() / a.norm()) <= tol[precision]
+
+
+# finest grids whose nested levels end in the tail: its top is an element level with explicit
+# rows (25 x 9, 33 x 31 and 31 x 33 nodes), or the level below it is already the coarsest
+NESTED = [(48, 16), (64, 60), (60, 64), (32, 8)]
+
+
+@pytest.mark.parametrize("nx,ny", NESTED)
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_tail_takes_element_levels(nx, ny, precision):
+    gp = gpu_problem(CANTILEVER, nx, ny)
+    gp.set_penalization(3)
+    xi = torch.as_tensor(smoothed_density(nx, ny, 6, sigma=2.0), device="cuda:0")
+    gen = torch.Generator(device="cpu").manual_seed(6)
+    r = torch.randn(2 * (nx + 1) * (ny + 1), generator=gen, dtype=torch.float64).cuda()
+    out = []
+    for tail in (0, 1):  # 0: the element level's own sweeps from its cell weights
+        gp.set_option("tail", tail)
+        out.append(gp.precondition(r, "elasticity", xi, precision=precision))
+    tol = {"fp64": 100 * 1.2e-16 * max(nx, ny) ** 2, "fp32": 1e-4}[precision]
+    assert float((out[0] - out[1]).norm() / out[0].norm()) <= tol

@@ -113,7 +113,8 @@ hipError_t elast_restrict_weights(int nxc, int nyc, const T* fine, T* coarse, hi
                                   float* coarse32 = nullptr);
 // explicit 9-point block stencil (BS=2, SoA: st[k*4+a*2+b][node]) of an element level
 template <typename T>
-hipError_t elast_to_stencil(const ElastOpArgs<T>& a, T* st, hipStream_t s);
+hipError_t elast_to_stencil(const ElastOpArgs<T>& a, T* st, hipStream_t s,
+                            float* st32 = nullptr);  // st32: also its FP32 copy
 
 // sensitivity rhs b_v = -p(1-m) sum_T e_T int_T xi^(p-1) lambda_v (P1)
 hipError_t elast_sensitivity(const SweepShape& sh, const double* xi, const double* u, int p,

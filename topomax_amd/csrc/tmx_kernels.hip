@@ -1017,7 +1017,7 @@ __device__ __forceinline__ void elast_to_stencil_body(const BlkId blk, const Ela
                                                       double hx,
                                                       double hy,
                                                       double lam,
-                                                      double mu) {
+                                                      double mu, float* st32) {
   const int nx = a.sh.nx, ny = a.sh.ny;
   const size_t nn = (size_t)(nx + 1) * (ny + 1);
   const size_t v = (size_t)blk.id * blockDim.x + threadIdx.x;
@@ -1081,24 +1081,29 @@ __device__ __forceinline__ void elast_to_stencil_body(const BlkId blk, const Ela
 #pragma unroll
   for (int kk = 0; kk < 9; ++kk)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) st[(size_t)(kk * 4 + e) * nn + v] = (T)acc[kk][e];
+    for (int e = 0; e < 4; ++e) {
+      st[(size_t)(kk * 4 + e) * nn + v] = (T)acc[kk][e];
+      if (st32) st32[(size_t)(kk * 4 + e) * nn + v] = (float)acc[kk][e];
+    }
 }
 
 template <typename T>
 __global__ void k_elast_to_stencil(ElastOpArgs<T> a, T* __restrict__ st,
-                                   double hx, double hy, double lam, double mu) {
-  elast_to_stencil_body<T>(hw_blk(), a, st, hx, hy, lam, mu);
+                                   double hx, double hy, double lam, double mu,
+                                   float* __restrict__ st32) {
+  elast_to_stencil_body<T>(hw_blk(), a, st, hx, hy, lam, mu, st32);
 }
 
 // lam, mu and a = hy/hx are recovered from the force constants (lam_h = l/2, mu_h = m/2,
 // mu_a = m a/2); the element matrices depend on hx, hy only through a.
 template <>
-hipError_t elast_to_stencil<double>(const ElastOpArgs<double>& a, double* st, hipStream_t s) {
+hipError_t elast_to_stencil<double>(const ElastOpArgs<double>& a, double* st, hipStream_t s,
+                                    float* st32) {
   // the constants are scale free (a = hy/hx); use hx = 1, hy = a.
   const double aa = a.k.mu_a / a.k.mu_h;  // = hy/hx
   const double mu = 2 * a.k.mu_h, lam = 2 * a.k.lam_h;
   const size_t nn = (size_t)(a.sh.nx + 1) * (a.sh.ny + 1);
-  TMX_LAUNCH_OR_RECORD(kBlock, (elast_to_stencil_body<double>), grid1d(nn), 0, s, (k_elast_to_stencil<double>), a, st, 1.0, aa, lam, mu);
+  TMX_LAUNCH_OR_RECORD(kBlock, (elast_to_stencil_body<double>), grid1d(nn), 0, s, (k_elast_to_stencil<double>), a, st, 1.0, aa, lam, mu, st32);
   return hipGetLastError();
 }
 

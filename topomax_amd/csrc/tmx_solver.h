@@ -105,6 +105,7 @@ struct Level {
   double hx = 0, hy = 0;
   int kind = kElem;
   int nested_from_prev = 0;  // transfer from level-1 to this level is nested P1
+  int rows = 0;              // element level with its explicit 9-point rows too (for the tail)
   size_t nn = 0;
   SweepShape sh64, sh32;
   // elasticity element levels > 0: per-cell (wA, wB)

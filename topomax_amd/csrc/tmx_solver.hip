@@ -93,9 +93,17 @@ int Hierarchy::init(Phys phys, int nx, int ny, double hx, double hy, unsigned fi
   L0.nn = (size_t)(nx + 1) * (ny + 1);
   levels_.push_back(std::move(L0));
   while (levels_.back().nn > (size_t)coarse_max_nodes) {
-    const Level& c = levels_.back();
+    Level& c = levels_.back();
     Level n;
-    if (c.kind == kElem && c.nx % 2 == 0 && c.ny % 2 == 0) {
+    // A coarser elasticity element level that fits the tail gets its explicit rows and the
+    // levels below it are bilinear, so that the tail runs all of them (one launch) where nested
+    // element levels would take two band launches of about 6.4 us each (whole FP64 steps: 60 x 20
+    // cells 2074 -> 1734 us, 320 x 160 2549 -> 2126, 640 x 320 3604 -> 3173; 32 designs 7821 ->
+    // 7269; iteration counts as before).  The filter's V-cycle, which only grids beyond its
+    // DCT solver use, keeps its element levels.
+    c.rows = phys == kElasticity && c.kind == kElem && levels_.size() > 1 &&
+             c.nn <= (size_t)kTailNodes;
+    if (c.kind == kElem && !c.rows && c.nx % 2 == 0 && c.ny % 2 == 0) {
       n.nx = c.nx / 2; n.ny = c.ny / 2; n.kind = kElem; n.nested_from_prev = 1;
     } else {
       n.nx = c.nx == 1 ? 1 : (c.nx + 1) / 2;
@@ -155,7 +163,8 @@ void Hierarchy::find_tail() {
   if (lastl >= 1 && bs_ * levels_[lastl].nn <= 128) {
     const size_t cap = (size_t)std::min(tail_nodes_, kTailNodes);
     int t = lastl;
-    while (t - 1 >= 1 && lastl - (t - 1) + 1 <= kMaxTail && levels_[t - 1].kind == kStencil &&
+    while (t - 1 >= 1 && lastl - (t - 1) + 1 <= kMaxTail &&
+           (levels_[t - 1].kind == kStencil || levels_[t - 1].rows) &&
            levels_[t - 1].nn <= cap && levels_[t].nn <= (size_t)kTailWg &&
            !levels_[t].nested_from_prev) {
       TailDims dims[kMaxTail];
@@ -258,12 +267,12 @@ int Hierarchy::alloc_vectors() {
       TMX_TRY(L.cw32.alloc(2 * (size_t)L.nx * L.ny));
     }
     const bool last = (l + 1 == levels_.size());
-    if (L.kind == kStencil || last) {
+    if (L.kind == kStencil || L.rows || last) {
       TMX_TRY(L.st64.alloc(9 * bs * bs * L.nn));
       TMX_TRY(L.st32.alloc(9 * bs * bs * L.nn));
     }
     // element level followed by a stencil level needs its explicit stencil for the RAP
-    if (L.kind == kElem && !last && levels_[l + 1].kind == kStencil)
+    if (L.kind == kElem && !L.rows && !last && levels_[l + 1].kind == kStencil)
       tmp_nodes = std::max(tmp_nodes, L.nn);
   }
   if (tmp_nodes) TMX_TRY(tmpst_.alloc(9 * bs * bs * tmp_nodes));
@@ -321,11 +330,13 @@ static ElastOpArgs<T> elast_args(const Hierarchy& h, int l, const T* xi, const T
 }
 
 // explicit stencil of element level l (fp64) into dst
-static int element_stencil(const Hierarchy& h, int l, double* dst, hipStream_t s) {
+// (dst32: elasticity, its FP32 copy)
+static int element_stencil(const Hierarchy& h, int l, double* dst, hipStream_t s,
+                           float* dst32 = nullptr) {
   const Level& L = h.levels_[l];
   if (h.phys_ == kElasticity) {
     ElastOpArgs<double> a = elast_args<double>(h, l, h.xi64_, L.cw64.get(), true, true);
-    TMX_HIP(elast_to_stencil<double>(a, dst, s));
+    TMX_HIP(elast_to_stencil<double>(a, dst, s, dst32));
   } else {
     TMX_HIP(filter_to_stencil<double>(L.nx, L.ny, FilterConst<double>::make(h.eps_, L.hx, L.hy),
                                       dst, s));
@@ -340,7 +351,10 @@ int Hierarchy::build_coarse_stencils(hipStream_t s) {
     Level& P = levels_[l - 1];
     if (L.kind == kStencil) {
       const double* src = nullptr;
-      if (P.kind == kElem) {
+      if (P.rows) {
+        TMX_TRY(element_stencil(*this, l - 1, P.st64.get(), s, P.st32.get()));
+        src = P.st64.get();
+      } else if (P.kind == kElem) {
         TMX_TRY(element_stencil(*this, l - 1, tmpst_.get(), s));
         src = tmpst_.get();
       } else {
@@ -404,9 +418,10 @@ int Hierarchy::update_elasticity(const double* xi, int p, double m, hipStream_t 
   for (int l = 1; l <= last; ++l) {
     Level& L = levels_[l];
     if (L.kind != kElem) {
-      first = l;
+      first = std::min(first, l);
       break;
     }
+    if (L.rows) first = l;
     const double* src = l == 1 ? cw0_.get() : levels_[l - 1].cw64.get();
     TMX_HIP(elast_restrict_weights<double>(L.nx, L.ny, src, L.cw64.get(), s, L.cw32.get()));
   }
