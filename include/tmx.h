@@ -237,10 +237,12 @@ enum tmx_option {
                                    node-row chunks of this height (default 12; tmx_autotune
                                    re-picks it per direction and precision); 0: the band
                                    kernels */
-  TMX_OPT_FILTER_DCT = 21,      /* 1 (default): the filter's preconditioner (FP32 and FP64) is
+  TMX_OPT_FILTER_DCT = 21,      /* 2 (default): the filter's preconditioner (FP32 and FP64) is
                                    the exact DCT-I / tridiagonal solver of
-                                   eps^2 K + (lumped mass) when ny is even and nx + 1 <= 3072
-                                   (3-5 PCG iterations); 0: the multigrid V-cycle */
+                                   eps^2 K + (lumped mass) where 2 ny has no prime factor above
+                                   350 (FP64) or 450 (FP32), ny <= 2048 and nx + 1 <= 3072
+                                   (3-5 PCG iterations); 1: only where 2 ny has no prime factor
+                                   above 7; 0: the multigrid V-cycle */
   TMX_OPT_PAIR_LEVELS = 22,     /* elasticity element levels 0 .. value-1 run the paired
                                    column-strip kernels, the levels below them the band kernels
                                    (default 1: the finest only); 1..8 */

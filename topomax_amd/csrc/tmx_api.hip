@@ -653,7 +653,7 @@ extern "C" int tmx_set_option(tmx_problem* h, int option, double value) {
       break;
     case TMX_OPT_FILTER_DCT:
       h->fl.drop_graphs();
-      h->fl.use_dct_ = value != 0.0;
+      h->fl.use_dct_ = value == 0.0 ? 0 : value == 2.0 ? 2 : 1;
       break;
     case TMX_OPT_PAIR_LEVELS:
       if (value < 1 || value > 8 || value != std::floor(value))

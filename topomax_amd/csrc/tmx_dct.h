@@ -21,8 +21,8 @@
 // (z[2n - j] = z[j]); the DFT of a real even sequence is real, so the real and imaginary parts
 // of the FFT are the two columns' transforms, up to the end-point terms
 //   T[m] = (Y[m] + r_0 + (-1)^m r_n) / 2,   Y = DFT_2n of the even extension.
-// The FFT is a mixed-radix Stockham transform (radices 2, 3, 4, 5, 7), so 2n must have no
-// prime factor above 7; other grids keep the multigrid V-cycle.
+// The FFT is a mixed-radix Stockham transform (radices 2, 3, 4, 5, 7, and direct sums for the
+// primes from 11 to kMaxPrime); other grids keep the multigrid V-cycle.
 #pragma once
 
 #include "tmx_kernels.h"
@@ -36,21 +36,33 @@ struct FftPlan {
   int L = 0;
   int nstages = 0;
   int radix[kMaxStages] = {};
+  bool direct = false;  // some radix has no butterfly of its own
 };
 
-// the radix plan of length L from radices {4, 2, 3, 5, 7}; false when L has a larger prime
-bool fft_plan(int L, FftPlan& plan);
+// the radix plan of length L: the prime factors above 7 first (none above max_prime; false when
+// there is one), then radices 4, 2, 3, 5, 7
+bool fft_plan(int L, int max_prime, FftPlan& plan);
 
 template <typename T>
 class DctPrecond {
  public:
-  // nx, ny: cells; 2 ny factors into 2, 3, 5, 7, nx + 1 <= kMaxRow, and the FFT of 2 ny
-  // points fits the LDS budget; eps: the filter's length scale
-  static bool supported(int nx, int ny);
+  // nx, ny: cells; 2 ny has no prime factor above max_prime (7 or kMaxPrime; above 7 on grids
+  // of more than kMinNodesDirect nodes only), nx + 1 <= kMaxRow, and the FFT of 2 ny points fits
+  // the LDS budget; eps: the filter's length scale
+  static bool supported(int nx, int ny, int max_prime);
   int init(int nx, int ny, double hx, double hy, double eps, hipStream_t s);
   // z = A'^-1 r (vectors of (nx + 1)(ny + 1) values), partials of r.z into rz if given
   int apply(const T* r, T* z, RedSlot* rz, hipStream_t s);
 
+  // Largest prime factor p of 2 ny: a prime without a butterfly costs p products per point
+  // (fft_stage_direct), the V-cycle the same per point whatever ny.  One filter solve to 1e-11,
+  // V-cycle / DCT in us: FP64 666 x 222 cells (p = 37) 978 / 304, 753 x 251 947 / 536, 933 x 311
+  // 974 / 791, 1203 x 401 1520 / 1646; FP32 954 / 275, 904 / 465, 907 / 662, 1377 / 1062 and
+  // 1503 x 503 1291 / 1392.
+  static constexpr int kMaxPrime = sizeof(T) == 4 ? 450 : 350;
+  // fewest nodes of a grid that such a prime's transform is used on: the V-cycle of a smaller
+  // one is a few launches (33 x 11 cells 296 / 413, 66 x 22 490 / 352)
+  static constexpr size_t kMinNodesDirect = 1024;
   // longest x row: one workgroup of 256 threads solves it, 12 rows per thread, with the row
   // and two coefficient arrays in LDS (40 KB in FP32, 80 KB in FP64 at this length)
   static constexpr int kMaxRow = 3072;

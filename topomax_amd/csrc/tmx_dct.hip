@@ -13,7 +13,7 @@
 
 namespace tmx {
 
-bool fft_plan(int L, FftPlan& plan) {
+bool fft_plan(int L, int max_prime, FftPlan& plan) {
   plan = FftPlan();
   plan.L = L;
   if (L < 2) return false;
@@ -24,6 +24,17 @@ bool fft_plan(int L, FftPlan& plan) {
     m /= r;
     return true;
   };
+  int rest = L;  // the primes above 7, largest stages first
+  for (int r : {2, 3, 5, 7})
+    while (rest % r == 0) rest /= r;
+  for (int r = 11; rest > 1; r += 2) {
+    if (r > max_prime) return false;
+    while (rest % r == 0) {
+      rest /= r;
+      plan.direct = true;
+      if (!push(r)) return false;
+    }
+  }
   while (m % 4 == 0)
     if (!push(4)) return false;
   while (m % 2 == 0)
@@ -169,12 +180,60 @@ __device__ __forceinline__ void fft_stage(V2<T>* buf, int L, int nseq, int Ns,
   __syncthreads();
 }
 
+// The same stage for a prime radix R without a butterfly of its own: each thread forms single
+// outputs, y_r = sum_k v_k exp(-2 pi i k r / R), R complex products each.  As the first stages
+// of the plan (Ns = 1 for the first), neighbouring lanes read neighbouring points and the same
+// twiddle, so a product costs two LDS reads.
+template <typename T, int NT>
+__device__ __forceinline__ void fft_stage_direct(V2<T>* buf, int L, int nseq, int Ns, int R,
+                                                 const V2<T>* __restrict__ tw) {
+  constexpr int MAXO = kFftMaxPoints / NT;
+  const int nb = L / R;
+  const int total = nseq * L;
+  const int span = L / (Ns * R);
+  const float ns_inv = 1.0f / (float)Ns, nb_inv = 1.0f / (float)nb;
+  V2<T> v[MAXO];
+  int dst[MAXO];
+#pragma unroll
+  for (int q = 0; q < MAXO; ++q) {
+    const int o = (int)threadIdx.x + q * NT;
+    dst[q] = -1;
+    if (o < total) {
+      const int f = o >= L ? 1 : 0;  // at most two sequences per workgroup
+      const int i = o - f * L;
+      const int r = div_fft(i, nb, nb_inv), j = i - r * nb;
+      const int jm = j - div_fft(j, Ns, ns_inv) * Ns;
+      const int step = jm * span + r * nb;  // < L
+      const V2<T>* src = buf + f * L + j;
+      V2<T> acc = src[0];
+      int k = step;
+#pragma unroll 4
+      for (int t = 1; t < R; ++t) {
+        const V2<T> a = src[t * nb], w = tw[k];
+        acc = {acc.x + (a.x * w.x - a.y * w.y), acc.y + (a.x * w.y + a.y * w.x)};
+        k += step;
+        if (k >= L) k -= L;
+      }
+      v[q] = acc;
+      dst[q] = f * L + (j - jm) * R + jm + r * Ns;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < MAXO; ++q)
+    if (dst[q] >= 0) buf[dst[q]] = v[q];
+  __syncthreads();
+}
+
 // DCT-I of the y-columns x0 .. x0 + C - 1 (x0 = C * group, C = 2 or 4), all n + 1 rows:
 //   dst[m][x] = sum_j src[j][x] cos(pi j m / n),  m = 0 .. n,
 // with (INV) partials of sum rdot . dst per workgroup.  Workgroups b, b + 8, b + 16, .. (one
 // XCD each, as workgroups are dealt out to the XCDs in turn) take consecutive column groups,
 // so the workgroups that share a row's cache line share that XCD's L2.
-template <typename T, bool INV, int C>
+// DIRECT: the plan has direct stages (a kernel of its own: they take the registers that set the
+// occupancy, 128 against 88 in FP32 and 175 against 152 in FP64: 32 designs 7388 us with one
+// kernel, 7196 with two).
+template <typename T, bool INV, int C, bool DIRECT>
 __device__ __forceinline__ void dct1_cols_body(const BlkId blk, int n, int mx, int groups,
                                                const FftPlan& plan, const V2<T>* tw_,
                                                const T* src_, T* dst_, const T* rdot_,
@@ -189,7 +248,8 @@ __device__ __forceinline__ void dct1_cols_body(const BlkId blk, int n, int mx, i
   V2<T>* z = reinterpret_cast<V2<T>*>(dct_lds);
   __shared__ V2<T> ends[2][2];  // each sequence's points 0 and n before the transform
   const int L = 2 * n;
-  V2<T>* twl = z + NS * L;  // the twiddle table, staged with the columns (FP32)
+  V2<T>* twl = z + NS * L;  // the twiddle table, staged with the columns (FP32, direct stages)
+  constexpr bool kStage = kTwiddlesInLds<T> || DIRECT;
   const int per = (int)blk.n / 8;
   const int g = ((int)blk.id % 8) * per + (int)blk.id / 8;
   double acc = 0.0;
@@ -201,7 +261,7 @@ __device__ __forceinline__ void dct1_cols_body(const BlkId blk, int n, int mx, i
     // at j and (0 < j < n) at its mirror L - j.  Eight loads in flight per thread.
     constexpr int NB = 8;
     constexpr int lc = C == 4 ? 2 : 1;  // log2 C
-    if (kTwiddlesInLds<T>)
+    if (kStage)
     for (int k0 = (int)threadIdx.x; k0 < L; k0 += 4 * NT) {
       V2<T> w[4];
 #pragma unroll
@@ -239,13 +299,16 @@ __device__ __forceinline__ void dct1_cols_body(const BlkId blk, int n, int mx, i
     int Ns = 1;
     for (int st = 0; st < plan.nstages; ++st) {
       const int R = plan.radix[st];
-      const V2<T>* twp = kTwiddlesInLds<T> ? static_cast<const V2<T>*>(twl) : tw;
+      const V2<T>* twp = kStage ? static_cast<const V2<T>*>(twl) : tw;
       switch (R) {
         case 2: fft_stage<T, 2, NT>(z, L, NS, Ns, twp); break;
         case 3: fft_stage<T, 3, NT>(z, L, NS, Ns, twp); break;
         case 4: fft_stage<T, 4, NT>(z, L, NS, Ns, twp); break;
         case 5: fft_stage<T, 5, NT>(z, L, NS, Ns, twp); break;
-        default: fft_stage<T, 7, NT>(z, L, NS, Ns, twp); break;
+        case 7: fft_stage<T, 7, NT>(z, L, NS, Ns, twp); break;
+        default:
+          if constexpr (DIRECT) fft_stage_direct<T, NT>(z, L, NS, Ns, R, twl);
+          break;
       }
       Ns *= R;
     }
@@ -288,7 +351,7 @@ __device__ __forceinline__ void dct1_cols_body(const BlkId blk, int n, int mx, i
   }
 }
 
-template <typename T, bool INV, int C>
+template <typename T, bool INV, int C, bool DIRECT>
 __global__ __launch_bounds__(kFftThreads<C>) void k_dct1_cols(int n, int mx, int groups,
                                                           FftPlan plan,
                                                           const V2<T>* __restrict__ tw,
@@ -296,21 +359,31 @@ __global__ __launch_bounds__(kFftThreads<C>) void k_dct1_cols(int n, int mx, int
                                                           T* __restrict__ dst,
                                                           const T* __restrict__ rdot,
                                                           double* __restrict__ part) {
-  dct1_cols_body<T, INV, C>(hw_blk(), n, mx, groups, plan, tw, src, dst, rdot, part);
+  dct1_cols_body<T, INV, C, DIRECT>(hw_blk(), n, mx, groups, plan, tw, src, dst, rdot, part);
 }
 
 // one DCT-I launch over the column groups (C = 2 or 4 columns per workgroup)
-template <typename T, bool INV>
-static void launch_dct1_cols(int cols, unsigned nblk, size_t lds, hipStream_t s, int n, int mx,
-                             int groups, const FftPlan& plan, const V2<T>* tw, const T* src,
-                             T* dst, const T* rdot, double* part) {
+template <typename T, bool INV, int C, bool DIRECT>
+static void launch_dct1_as(unsigned nblk, size_t lds, hipStream_t s, int n, int mx, int groups,
+                           const FftPlan& plan, const V2<T>* tw, const T* src, T* dst,
+                           const T* rdot, double* part) {
+  TMX_LAUNCH_OR_RECORD(kFftThreads<C>, (dct1_cols_body<T, INV, C, DIRECT>), nblk, lds, s,
+                       (k_dct1_cols<T, INV, C, DIRECT>), n, mx, groups, plan, tw, src, dst, rdot,
+                       part);
+}
+
+template <typename T, bool INV, typename... A>
+static void launch_dct1_cols(int cols, const FftPlan& plan, unsigned nblk, size_t lds,
+                             hipStream_t s, int n, int mx, int groups, A... a) {
   if constexpr (sizeof(T) == 4) {  // (FP64 always takes two columns)
     if (cols == 4) {
-      TMX_LAUNCH_OR_RECORD(kFftThreads<4>, (dct1_cols_body<T, INV, 4>), nblk, lds, s, (k_dct1_cols<T, INV, 4>), n, mx, groups, plan, tw, src, dst, rdot, part);
+      if (plan.direct) launch_dct1_as<T, INV, 4, true>(nblk, lds, s, n, mx, groups, plan, a...);
+      else launch_dct1_as<T, INV, 4, false>(nblk, lds, s, n, mx, groups, plan, a...);
       return;
     }
   }
-  TMX_LAUNCH_OR_RECORD(kFftThreads<2>, (dct1_cols_body<T, INV, 2>), nblk, lds, s, (k_dct1_cols<T, INV, 2>), n, mx, groups, plan, tw, src, dst, rdot, part);
+  if (plan.direct) launch_dct1_as<T, INV, 2, true>(nblk, lds, s, n, mx, groups, plan, a...);
+  else launch_dct1_as<T, INV, 2, false>(nblk, lds, s, n, mx, groups, plan, a...);
 }
 
 // One tridiagonal solve along x per mode row: row m of `modes` is mode m (workgroup m).  Each
@@ -479,8 +552,9 @@ __global__ __launch_bounds__(kTriThreads) void k_dct_tri(int mx, int n, T a_off,
 // LDS of k_dct1_cols: the complex sequences of `cols` columns (2 n points each per pair) and
 // the twiddle table of 2 n points
 template <typename T>
-static size_t dct_cols_lds(int cols, int n) {
-  return ((size_t)(cols / 2) + (kTwiddlesInLds<T> ? 1 : 0)) * 2 * (size_t)n * sizeof(V2<T>);
+static size_t dct_cols_lds(int cols, int n, bool direct) {
+  return ((size_t)(cols / 2) + (kTwiddlesInLds<T> || direct ? 1 : 0)) * 2 * (size_t)n *
+         sizeof(V2<T>);
 }
 
 // columns per FFT workgroup: in FP32 four (two complex sequences, 16-byte row segments, on
@@ -490,22 +564,24 @@ static size_t dct_cols_lds(int cols, int n) {
 template <typename T>
 static int dct_cols(int n) {
   return sizeof(T) == 4 && n >= 512 && (4 / 2) * 2 * n <= kFftMaxPoints &&
-                 dct_cols_lds<T>(4, n) <= 64 * 1024
+                 dct_cols_lds<T>(4, n, false) <= 64 * 1024
              ? 4
              : 2;
 }
 
 template <typename T>
-bool DctPrecond<T>::supported(int nx, int ny) {
+bool DctPrecond<T>::supported(int nx, int ny, int max_prime) {
   FftPlan p;
-  return ny >= 1 && nx >= 1 && nx + 1 <= kMaxRow && fft_plan(2 * ny, p) &&
-         (kCols / 2) * 2 * ny <= kFftMaxPoints;
+  return ny >= 1 && nx >= 1 && nx + 1 <= kMaxRow && (kCols / 2) * 2 * ny <= kFftMaxPoints &&
+         fft_plan(2 * ny, max_prime, p) &&
+         (!p.direct || (size_t)(nx + 1) * (ny + 1) > kMinNodesDirect);
 }
 
 template <typename T>
 int DctPrecond<T>::init(int nx, int ny, double hx, double hy, double eps, hipStream_t s) {
-  if (!supported(nx, ny)) {
-    set_error("internal: DCT preconditioner needs 2 ny with prime factors <= 7, ny <= " +
+  if (!supported(nx, ny, kMaxPrime)) {
+    set_error("internal: DCT preconditioner needs 2 ny with prime factors <= " +
+              std::to_string(kMaxPrime) + ", ny <= " +
               std::to_string(kFftMaxPoints / kCols) + " and nx + 1 <= " +
               std::to_string(kMaxRow));
     return -1;
@@ -517,7 +593,7 @@ int DctPrecond<T>::init(int nx, int ny, double hx, double hy, double eps, hipStr
   hy_ = hy;
   eps_ = eps;
   const int L = 2 * ny;
-  (void)fft_plan(L, plan_);
+  (void)fft_plan(L, kMaxPrime, plan_);
   // twiddles exp(-2 pi i k / L) from the exact integer angle, evaluated in double
   std::vector<T> tw(2 * (size_t)L);
   for (int k = 0; k < L; ++k) {
@@ -533,15 +609,20 @@ int DctPrecond<T>::init(int nx, int ny, double hx, double hy, double eps, hipStr
   TMX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_dct_tri<T>),
                               hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)dct_tri_lds<T>(kMaxRow)));
-  std::vector<const void*> fns = {reinterpret_cast<const void*>(&k_dct1_cols<T, false, 2>),
-                                   reinterpret_cast<const void*>(&k_dct1_cols<T, true, 2>)};
+  auto raise_lds = [&](const void* f, bool direct) {
+    return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)dct_cols_lds<T>(kCols, kFftMaxPoints / 2, direct));
+  };
+  TMX_HIP(raise_lds(reinterpret_cast<const void*>(&k_dct1_cols<T, false, 2, false>), false));
+  TMX_HIP(raise_lds(reinterpret_cast<const void*>(&k_dct1_cols<T, true, 2, false>), false));
+  TMX_HIP(raise_lds(reinterpret_cast<const void*>(&k_dct1_cols<T, false, 2, true>), true));
+  TMX_HIP(raise_lds(reinterpret_cast<const void*>(&k_dct1_cols<T, true, 2, true>), true));
   if constexpr (sizeof(T) == 4) {
-    fns.push_back(reinterpret_cast<const void*>(&k_dct1_cols<T, false, 4>));
-    fns.push_back(reinterpret_cast<const void*>(&k_dct1_cols<T, true, 4>));
+    TMX_HIP(raise_lds(reinterpret_cast<const void*>(&k_dct1_cols<T, false, 4, false>), false));
+    TMX_HIP(raise_lds(reinterpret_cast<const void*>(&k_dct1_cols<T, true, 4, false>), false));
+    TMX_HIP(raise_lds(reinterpret_cast<const void*>(&k_dct1_cols<T, false, 4, true>), true));
+    TMX_HIP(raise_lds(reinterpret_cast<const void*>(&k_dct1_cols<T, true, 4, true>), true));
   }
-  for (const void* f : fns)
-    TMX_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)dct_cols_lds<T>(kCols, kFftMaxPoints / 2)));
   return 0;
 }
 
@@ -551,11 +632,12 @@ int DctPrecond<T>::apply(const T* r, T* z, RedSlot* rz, hipStream_t s) {
   const int cols = dct_cols<T>(n);
   const int groups = (mx + cols - 1) / cols;
   const int nblk = 8 * ((groups + 7) / 8);
-  const size_t lds = dct_cols_lds<T>(cols, n);
+  const size_t lds = dct_cols_lds<T>(cols, n, plan_.direct);
   const V2<T>* tw = reinterpret_cast<const V2<T>*>(tw_.get());
   T* t = t_.get();
   // forward DCT-I along y: t[m] = sum_j r[j] cos(pi j m / n)
-  launch_dct1_cols<T, false>(cols, nblk, lds, s, n, mx, groups, plan_, tw, r, t, nullptr, nullptr);
+  launch_dct1_cols<T, false>(cols, plan_, nblk, lds, s, n, mx, groups, tw, r, t,
+                             static_cast<const T*>(nullptr), static_cast<double*>(nullptr));
   TMX_HIP(hipGetLastError());
   // tridiagonal solves along x, one workgroup per mode (scaled by 1 / D_m there)
   const T a_off = (T)(eps_ * eps_ * hy_ / hx_);
@@ -572,7 +654,8 @@ int DctPrecond<T>::apply(const T* r, T* z, RedSlot* rz, hipStream_t s) {
     rz->nblocks = nblk;
     part = rz->partials;
   }
-  launch_dct1_cols<T, true>(cols, nblk, lds, s, n, mx, groups, plan_, tw, t, z, r, part);
+  launch_dct1_cols<T, true>(cols, plan_, nblk, lds, s, n, mx, groups, tw,
+                            static_cast<const T*>(t), z, r, part);
   TMX_HIP(hipGetLastError());
   return 0;
 }

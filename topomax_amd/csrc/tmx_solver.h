@@ -326,7 +326,8 @@ class Hierarchy {
   int fpipe_rows_[2][2] = {{12, 12}, {12, 12}};
   // filter preconditioner: the exact DCT-I / tridiagonal solver of the tensor-lumped
   // operator (tmx_dct.h) instead of the V-cycle, where the grid allows it
-  bool use_dct_ = true;
+  // (0: never, 1: only where 2 ny has no prime factor above 7, 2: with larger primes too)
+  int use_dct_ = 2;
   std::unique_ptr<DctPrecond<float>> dct32_;
   std::unique_ptr<DctPrecond<double>> dct64_;
   template <typename T>

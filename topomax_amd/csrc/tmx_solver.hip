@@ -735,7 +735,8 @@ int Hierarchy::vcycle(int l, const T* b, T* out, hipStream_t s, RedSlot* dot_bz)
   }
   if (use_tail_ && l == tail_ && l > 0) return tail_launch<T>(*this, b, out, s);
   if (l == 0 && phys_ == kFilter && use_dct_ && !use_graphs_ &&
-      DctPrecond<T>::supported(levels_[0].nx, levels_[0].ny)) {
+      DctPrecond<T>::supported(levels_[0].nx, levels_[0].ny,
+                               use_dct_ == 1 ? 7 : DctPrecond<T>::kMaxPrime)) {
     auto& dct = dct_slot<T>();
     if (!dct) {
       std::unique_ptr<DctPrecond<T>> d(new DctPrecond<T>);
