@@ -218,7 +218,7 @@ enum tmx_option {
                                    kernels too */
   TMX_OPT_FINE_CELL_WEIGHTS = 15, /* elasticity finest-level V-cycle sweeps read per-cell
                                    weights formed once per operator instead of the nodal xi:
-                                   bit 0 FP32 V-cycles (default on), bit 1 FP64 */
+                                   bit 0 FP32 V-cycles, bit 1 FP64 (both on by default) */
   TMX_OPT_GRAPHS = 16,          /* 1: PCG iterations replay captured hipGraphs; 0 (default):
                                    their kernels are launched one by one (measured faster) */
   TMX_OPT_SWEEP_PAIRS = 17,     /* > 0: the elasticity finest level runs its first two
