@@ -164,7 +164,7 @@ def instep_kernel_us(problem, rho, steps, precision, rtol, kernel=ROOFLINE_KERNE
 
 def p2_throughput(N: int, steps: int, rtol: float, mixed: bool = True):
     """The reference's own element (P2 displacement, FEM_src/elasisity_problem.py:194-196) on
-    the same cantilever at N: FP64 MINRES preconditioned by P2 block Jacobi over the P1
+    the same cantilever at N: FP64 PCG preconditioned by P2 block Jacobi over the P1
     multigrid, one objective + gradient per step; with mixed, also the same solve with the
     preconditioner's P1 V-cycle in FP32 (precision "mixed")."""
     import torch

@@ -89,8 +89,8 @@ typedef struct tmx_problem_desc {
   int degree;                 /* displacement element: 1 (P1, default when 0) or 2 (P2, the
                                  reference's VectorElement("CG", triangle, 2),
                                  FEM_src/elasisity_problem.py:194-196); P2 solves run in FP64
-                                 (MINRES preconditioned by P2 block Jacobi over the P1
-                                 multigrid) and u has 2 (2nx+1)(2ny+1) entries */
+                                 (PCG, MINRES where K is indefinite, preconditioned by P2
+                                 block Jacobi over the P1 multigrid) and u has 2 (2nx+1)(2ny+1) entries */
 } tmx_problem_desc;
 
 typedef struct tmx_solve_opts {

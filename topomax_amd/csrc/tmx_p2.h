@@ -49,6 +49,16 @@ hipError_t p2_smooth_first32(const P2Geom& g, const float* W, const float* D, co
                              float* b32, float* y, double omega, hipStream_t s);
 hipError_t p2_smooth_last32(const P2Geom& g, const float* W, const float* D, const float* x,
                             const float* b, double* y, double omega, hipStream_t s);
+// a sweep (x not null) with the partials of b.y; TB = double with T = float reads a double b
+template <typename T, typename TB>
+hipError_t p2_smooth_dot(const P2Geom& g, const T* W, const T* D, const T* x, const TB* b, T* y,
+                         double omega, RedSlot* by, hipStream_t s);
+// PCG's direction update and operator step in one launch: p_new = z + (*beta) p_old, q = K p_new
+// with the partials of p_new.q, and x += (*alpha) p_old (p_old, z zero on fixed nodes)
+template <typename TZ>
+hipError_t p2_apply_update(const P2Geom& g, const double* W, const double* p_old, const TZ* z,
+                           double* p_new, double* q, double* x, const double* beta,
+                           const double* alpha, RedSlot* pq, hipStream_t s);
 // r = b - K x
 template <typename T>
 hipError_t p2_residual(const P2Geom& g, const T* W, const T* x, const T* b, T* r, hipStream_t s);

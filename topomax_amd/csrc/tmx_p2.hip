@@ -279,7 +279,11 @@ __global__ void k_p2_weights(P2Geom g, const double* __restrict__ xi, int p, dou
 //   MODE 0: y = K u (fixed nodes: y = u);  1: y = b - K u (fixed: b - u);
 //   2: y = x + omega D^-1 (b - K x) (x null: from zero; fixed nodes 0);
 //   3: MINRES's operator step y = K u - (*mb / *mo) b (0 when *mo is 0), with the partial of
-//      u.y of the workgroup's owned nodes in part[workgroup] (FP64).
+//      u.y of the workgroup's owned nodes in part[workgroup] (FP64);
+//   4: PCG's direction update and operator step (FP64): u = b + (*mb) x (b: z, x: the old
+//      direction), written to ynew, y = K u with the partial of u.y in part, and the previous
+//      iteration's deferred iterate update xk += (*mo) x.  Fixed nodes hold zeros throughout.
+//   In mode 2 with part, the partial of b.y (both as read and written).
 // T: FP64, or FP32 for the mixed scheme's preconditioner (weights, diagonal blocks and vectors
 // in float, the diagonal blocks inverted by the hardware reciprocal).  TB / TY: the types of b
 // and y (a double right-hand side read, or a double result written, by the float cycle's
@@ -359,7 +363,9 @@ __global__ __launch_bounds__(kP2TileThreads) void k_p2_tile(P2Geom g, const T* _
                                                             T* __restrict__ bcopy = nullptr,
                                                             const double* __restrict__ mb = nullptr,
                                                             const double* __restrict__ mo = nullptr,
-                                                            double* __restrict__ part = nullptr) {
+                                                            double* __restrict__ part = nullptr,
+                                                            T* __restrict__ ynew = nullptr,
+                                                            T* __restrict__ xk = nullptr) {
   __shared__ T us[kP2ExtN * kP2ExtN][2];
   __shared__ T fs[kP2ExtC * kP2ExtC][2][6][2];
   const int nX = 2 * g.nx + 1, nY = 2 * g.ny + 1;
@@ -368,6 +374,11 @@ __global__ __launch_bounds__(kP2TileThreads) void k_p2_tile(P2Geom g, const T* _
   const int Y0 = (int)(blockIdx.x / (unsigned)ntx) * kP2TileC;
   const int LI0 = 2 * X0 - 2, LJ0 = 2 * Y0 - 2;  // lattice origin of the staged region
   const bool forces = MODE != 2 || x != nullptr;
+  T cg_beta = T(0), cg_alpha = T(0);
+  if constexpr (MODE == 4) {
+    cg_beta = *mb;
+    cg_alpha = *mo;
+  }
   if (forces) {
     for (int k = (int)threadIdx.x; k < kP2ExtN * kP2ExtN; k += kP2TileThreads) {
       const int lj = k / kP2ExtN, li = k - lj * kP2ExtN;
@@ -377,6 +388,10 @@ __global__ __launch_bounds__(kP2TileThreads) void k_p2_tile(P2Geom g, const T* _
         const size_t n = (size_t)J * nX + I;
         u0 = x[2 * n];
         u1 = x[2 * n + 1];
+        if constexpr (MODE == 4) {
+          u0 = (T)b[2 * n] + cg_beta * u0;
+          u1 = (T)b[2 * n + 1] + cg_beta * u1;
+        }
       }
       us[k][0] = u0;
       us[k][1] = u1;
@@ -412,7 +427,7 @@ __global__ __launch_bounds__(kP2TileThreads) void k_p2_tile(P2Geom g, const T* _
   const int IE = X0 + kP2TileC >= g.nx ? nX : 2 * (X0 + kP2TileC);
   const int JE = Y0 + kP2TileC >= g.ny ? nY : 2 * (Y0 + kP2TileC);
   const int OW = IE - 2 * X0, OH = JE - 2 * Y0;
-  double dot_part = 0.0;  // (MODE 3)
+  double dot_part = 0.0;
   double cl = 0.0;
   if constexpr (MODE == 3) cl = *mo != 0.0 ? *mb / *mo : 0.0;
   for (int k = (int)threadIdx.x; k < OW * OH; k += kP2TileThreads) {
@@ -438,6 +453,16 @@ __global__ __launch_bounds__(kP2TileThreads) void k_p2_tile(P2Geom g, const T* _
       y[2 * n] = y0;
       y[2 * n + 1] = y1;
       dot_part += u0 * y0 + u1 * y1;
+    } else if constexpr (MODE == 4) {
+      const int li = (I - LI0) + (J - LJ0) * kP2ExtN;
+      const T u0 = us[li][0], u1 = us[li][1];
+      y[2 * n] = f0;
+      y[2 * n + 1] = f1;
+      ynew[2 * n] = u0;
+      ynew[2 * n + 1] = u1;
+      xk[2 * n] += cg_alpha * x[2 * n];
+      xk[2 * n + 1] += cg_alpha * x[2 * n + 1];
+      dot_part += u0 * f0 + u1 * f1;
     } else if constexpr (MODE == 1) {
       y[2 * n] = b[2 * n] - (fx ? x[2 * n] : f0);
       y[2 * n + 1] = b[2 * n + 1] - (fx ? x[2 * n + 1] : f1);
@@ -454,12 +479,15 @@ __global__ __launch_bounds__(kP2TileThreads) void k_p2_tile(P2Geom g, const T* _
         const T a = D[3 * n], c = D[3 * n + 1], e = D[3 * n + 2];
         const T inv = recip(a * e - c * c);
         const T x0 = x ? x[2 * n] : T(0), x1 = x ? x[2 * n + 1] : T(0);
-        y[2 * n] = (TY)(x0 + omega * (e * rx - c * ry) * inv);
-        y[2 * n + 1] = (TY)(x1 + omega * (a * ry - c * rx) * inv);
+        const T y0 = x0 + omega * (e * rx - c * ry) * inv;
+        const T y1 = x1 + omega * (a * ry - c * rx) * inv;
+        y[2 * n] = (TY)y0;
+        y[2 * n + 1] = (TY)y1;
+        dot_part += (double)b[2 * n] * (double)y0 + (double)b[2 * n + 1] * (double)y1;
       }
     }
   }
-  if constexpr (MODE == 3) {
+  if (MODE >= 3 || (MODE == 2 && part)) {
     const double vv[1] = {dot_part};
     double* const o[1] = {part};
     block_partials<1, kP2TileThreads>(vv, o, blockIdx.x);
@@ -714,6 +742,42 @@ hipError_t p2_diag(const P2Geom& g, const double* W, double* D, hipStream_t s) {
   k_p2_diag<<<grid_for(g.nodes()), 256, 0, s>>>(g, W, D);
   return hipGetLastError();
 }
+
+template <typename T, typename TB>
+hipError_t p2_smooth_dot(const P2Geom& g, const T* W, const T* D, const T* x, const TB* b, T* y,
+                         double omega, RedSlot* by, hipStream_t s) {
+  if (!D || !x || !b || !y || !by || p2_tiles(g) > (unsigned)kMaxPartials)
+    return hipErrorInvalidValue;
+  by->nblocks = (int)p2_tiles(g);
+  k_p2_tile<2, T, TB, T><<<p2_tiles(g), kP2TileThreads, 0, s>>>(
+      g, W, D, x, b, y, (T)omega, nullptr, nullptr, nullptr, by->partials);
+  return hipGetLastError();
+}
+template hipError_t p2_smooth_dot<double, double>(const P2Geom&, const double*, const double*,
+                                                  const double*, const double*, double*, double,
+                                                  RedSlot*, hipStream_t);
+template hipError_t p2_smooth_dot<float, double>(const P2Geom&, const float*, const float*,
+                                                 const float*, const double*, float*, double,
+                                                 RedSlot*, hipStream_t);
+
+template <typename TZ>
+hipError_t p2_apply_update(const P2Geom& g, const double* W, const double* p_old, const TZ* z,
+                           double* p_new, double* q, double* x, const double* beta,
+                           const double* alpha, RedSlot* pq, hipStream_t s) {
+  if (!p_old || !z || !p_new || !q || !x || !beta || !alpha || !pq ||
+      p2_tiles(g) > (unsigned)kMaxPartials)
+    return hipErrorInvalidValue;
+  pq->nblocks = (int)p2_tiles(g);
+  k_p2_tile<4, double, TZ, double><<<p2_tiles(g), kP2TileThreads, 0, s>>>(
+      g, W, nullptr, p_old, z, q, 0.0, nullptr, beta, alpha, pq->partials, p_new, x);
+  return hipGetLastError();
+}
+template hipError_t p2_apply_update<double>(const P2Geom&, const double*, const double*,
+                                            const double*, double*, double*, double*,
+                                            const double*, const double*, RedSlot*, hipStream_t);
+template hipError_t p2_apply_update<float>(const P2Geom&, const double*, const double*,
+                                           const float*, double*, double*, double*, const double*,
+                                           const double*, RedSlot*, hipStream_t);
 
 template <typename T>
 hipError_t p2_smooth(const P2Geom& g, const T* W, const T* D, const T* x, const T* b, T* y,

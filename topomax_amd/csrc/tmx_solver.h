@@ -154,6 +154,16 @@ struct SolveStats {
   void complete();
 };
 
+// The host side of one PCG solve whose start has been queued (host_bb set to NaN before it):
+// queues the iterations by launch(k), k = 1, 2, .., whose finalize reports into the ring slot of
+// their parity, one ahead of the one it waits for, until one reports that it stopped;
+// end(launched, gated) queues the deferred x += alpha p of iteration `launched` (pcg_enqueue_end).
+// gate: queue that gated on the stop flag whenever nothing is queued behind the awaited one.
+int pcg_drive(Workspace& ws, size_t n, const char* what, double rtol, int max_iter, bool gate,
+              const std::function<int(int)>& launch,
+              const std::function<int(int, bool)>& end, double* bnorm2, int* iters, double* rel,
+              hipStream_t s);
+
 // Preconditioned MINRES (FP64) on A x = b from x0 = 0, restarted on the true residual until
 // |b - A x| <= rtol |b|.  apply(x, y): y = A x.  precond(r, z, rz): z = M^-1 r with M SPD and
 // the partials of r.z in rz.  bufs: eight vectors of n doubles (two residuals, two work

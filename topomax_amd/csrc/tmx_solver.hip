@@ -1040,25 +1040,14 @@ int Hierarchy::pcg_enqueue_end(Workspace& ws, int launched, hipStream_t s, bool 
   return 0;
 }
 
-template <typename T, typename PC>
-int Hierarchy::pcg(Workspace& ws, const T* b, double rtol, int max_iter, double* bnorm2,
-                   int* iters, double* rel, hipStream_t s) {
-  const size_t nv = n();
-  const int prec = !std::is_same<T, PC>::value ? 2 : sizeof(T) == 8 ? 0 : 1;
-  if (graphs_cw0_ != has_cw0_) drop_graphs();  // captured with the other finest-level source
-  graphs_cw0_ = has_cw0_;
-  if (use_graphs_)
-    for (int w = 0; w < 3; ++w)
-      if (!graphs_[prec][w]) TMX_TRY((capture<T, PC>(*this, ws, w, &graphs_[prec][w], s)));
+int pcg_drive(Workspace& ws, size_t n, const char* what, double rtol, int max_iter, bool gate,
+              const std::function<int(int)>& launch,
+              const std::function<int(int, bool)>& end, double* bnorm2, int* iters, double* rel,
+              hipStream_t s) {
+  volatile double* host_bb = ws.host + Workspace::kScalars + kRingBB;
   *iters = 0;
   *rel = 1.0;
-  // r = b, x = 0 (and the float r of a mixed V-cycle) with |b|^2, the tolerance and the start
-  // flag formed on the device: no host round trip before the first iteration
-  volatile double* host_bb = ws.host + Workspace::kScalars + kRingBB;
-  host_bb[0] = std::numeric_limits<double>::quiet_NaN();
-  TMX_TRY((pcg_enqueue_begin<T, PC>(ws, b, rtol, !use_graphs_, s)));
-  if (use_graphs_) TMX_HIP(hipGraphLaunch(graphs_[prec][0], s));
-  // Iteration k runs graph 1 + (k-1)%2, whose last kernel writes (flag, r.r, iterations) and
+  // launch(k) queues iteration k, whose last kernel writes (flag, r.r, iterations) and
   // then the sequence number k to ring slot (k-1)%2 in pinned host memory; the host polls that
   // number (no event packets between the graphs).  While the host waits for iteration k it
   // normally has iteration k+1 queued already, so the device never idles.  An iteration queued
@@ -1071,11 +1060,6 @@ int Hierarchy::pcg(Workspace& ws, const T* b, double rtol, int max_iter, double*
   // no PCG iteration of this stream is in flight: an earlier solve returned only after every
   // iteration it queued had reported
   ring[3] = ring[7] = 0.0;
-  auto launch = [&](int k) -> hipError_t {
-    if (use_graphs_) return hipGraphLaunch(graphs_[prec][1 + ((k - 1) & 1)], s);
-    if (enqueue_pcg_iteration<T, PC>(*this, ws, (k - 1) & 1, s) != 0) return hipErrorUnknown;
-    return hipSuccess;
-  };
   // wait until iteration k has reported; a stream that drains without the report is an error,
   // never a hang
   auto wait_iter = [&](int k) -> int {
@@ -1103,16 +1087,16 @@ int Hierarchy::pcg(Workspace& ws, const T* b, double rtol, int max_iter, double*
   // round trip; unconverged, it changes nothing and the next iteration applies the update.
   int gated = 0;
   if (max_iter >= 1) {
-    TMX_HIP(launch(1));
+    TMX_TRY(launch(1));
     launched = 1;
   }
   while (done < launched) {
     if (launched == done + 1 && launched < max_iter && !near) {
-      TMX_HIP(launch(launched + 1));
+      TMX_TRY(launch(launched + 1));
       ++launched;
     }
-    if (launched == done + 1 && gate_end_) {
-      TMX_TRY(pcg_enqueue_end<T>(ws, launched, s, true));
+    if (launched == done + 1 && gate) {
+      TMX_TRY(end(launched, true));
       gated = launched;
     }
     TMX_TRY(wait_iter(done + 1));
@@ -1129,7 +1113,7 @@ int Hierarchy::pcg(Workspace& ws, const T* b, double rtol, int max_iter, double*
     rr_last = rr;
     near = rr * std::min(ratio, 1.0) <= 4.0 * tol2;
     if (launched == done && done < max_iter) {
-      TMX_HIP(launch(done + 1));
+      TMX_TRY(launch(done + 1));
       ++launched;
     }
   }
@@ -1137,7 +1121,7 @@ int Hierarchy::pcg(Workspace& ws, const T* b, double rtol, int max_iter, double*
   // host waits for the last queued iteration's report, so the device does not idle meanwhile
   // (already queued when the gated update of the last iteration found its stop flag set)
   if (launched > 0 && !(gated == launched && done == launched && flag != 0.0))
-    TMX_TRY(pcg_enqueue_end<T>(ws, launched, s));
+    TMX_TRY(end(launched, false));
   if (launched > done) TMX_TRY(wait_iter(launched));
   if (launched == 0) {  // no iteration reported |b|^2: read it
     TMX_TRY(ws.read(s, kScBB, 1));
@@ -1151,9 +1135,8 @@ int Hierarchy::pcg(Workspace& ws, const T* b, double rtol, int max_iter, double*
   *iters = launched > 0 ? (int)slot(launched)[2] : 0;
   *rel = bb > 0.0 ? std::sqrt(std::max(rrv, 0.0) / bb) : 0.0;
   if (g_trace)
-    std::fprintf(stderr, "[tmx] pcg<%s> %s n=%zu: %d its, rel %.3e, flag %g\n",
-                 prec == 2 ? "f64/f32" : prec == 0 ? "f64" : "f32", phys_ == kElasticity ? "elast" : "filter", nv,
-                 *iters, *rel, flag);
+    std::fprintf(stderr, "[tmx] pcg %s n=%zu: %d its, rel %.3e, flag %g\n", what, n, *iters, *rel,
+                 flag);
   if (flag == 1.0) return 0;
   if (flag == 2.0) {
     set_error("PCG breakdown: p.Ap <= 0 (operator not positive definite)");
@@ -1165,6 +1148,33 @@ int Hierarchy::pcg(Workspace& ws, const T* b, double rtol, int max_iter, double*
   }
   set_error("PCG did not reach the tolerance within the iteration limit");
   return -3;
+}
+
+template <typename T, typename PC>
+int Hierarchy::pcg(Workspace& ws, const T* b, double rtol, int max_iter, double* bnorm2,
+                   int* iters, double* rel, hipStream_t s) {
+  const int prec = !std::is_same<T, PC>::value ? 2 : sizeof(T) == 8 ? 0 : 1;
+  if (graphs_cw0_ != has_cw0_) drop_graphs();  // captured with the other finest-level source
+  graphs_cw0_ = has_cw0_;
+  if (use_graphs_)
+    for (int w = 0; w < 3; ++w)
+      if (!graphs_[prec][w]) TMX_TRY((capture<T, PC>(*this, ws, w, &graphs_[prec][w], s)));
+  // r = b, x = 0 (and the float r of a mixed V-cycle) with |b|^2, the tolerance and the start
+  // flag formed on the device: no host round trip before the first iteration
+  volatile double* host_bb = ws.host + Workspace::kScalars + kRingBB;
+  host_bb[0] = std::numeric_limits<double>::quiet_NaN();
+  TMX_TRY((pcg_enqueue_begin<T, PC>(ws, b, rtol, !use_graphs_, s)));
+  if (use_graphs_) TMX_HIP(hipGraphLaunch(graphs_[prec][0], s));
+  auto launch = [&](int k) -> int {
+    if (use_graphs_) TMX_HIP(hipGraphLaunch(graphs_[prec][1 + ((k - 1) & 1)], s));
+    else TMX_TRY((enqueue_pcg_iteration<T, PC>(*this, ws, (k - 1) & 1, s)));
+    return 0;
+  };
+  auto end = [&](int launched, bool gated) { return pcg_enqueue_end<T>(ws, launched, s, gated); };
+  const char* what = phys_ == kElasticity
+                         ? (prec == 2 ? "f64/f32 elast" : prec == 0 ? "f64 elast" : "f32 elast")
+                         : (prec == 2 ? "f64/f32 filter" : prec == 0 ? "f64 filter" : "f32 filter");
+  return pcg_drive(ws, n(), what, rtol, max_iter, gate_end_, launch, end, bnorm2, iters, rel, s);
 }
 
 // Reliable-update PCG iteration: the FP32 Krylov iteration of enqueue_pcg_iteration<float>
