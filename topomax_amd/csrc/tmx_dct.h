@@ -1,20 +1,27 @@
-// Exact fast solver of the filter's spectrally equivalent operator, used as its PCG
+// Exact fast solver of a spectrally equivalent operator of the filter, used as its PCG
 // preconditioner (FP32 in the mixed scheme, FP64 in the FP64 scheme).
 //
 // With natural boundary conditions on the structured 'right' mesh the filter stiffness is a
 // sum of Kronecker products of 1D Neumann Laplacians T (tridiag(-1, 2, -1), boundary diagonal
 // 1) with the boundary half-weights W = diag(1/2, 1, ..., 1, 1/2):
 //   eps^2 K = eps^2 (hy/hx) W_y (x) T_x + eps^2 (hx/hy) T_y (x) W_x   (y outer, x inner).
-// Replacing the consistent mass by hx hy W_y (x) W_x gives
-//   A' = W_y (x) B_x + T_y (x) C_x,  B_x = eps^2 (hy/hx) T_x + hx hy W_x,  C_x = eps^2 (hx/hy) W_x,
-// which the DCT-I in y diagonalises: T_y v_m = lambda_m W_y v_m with v_m[j] = cos(pi j m / n),
-// lambda_m = 2 - 2 cos(pi m / n), v_m' W_y v_k = D_m delta_mk (D_m = n / 2, or n for m = 0, n).
-// So A'^-1 r = sum_m v_m (x) (B_x + lambda_m C_x)^-1 (v_m' r) / D_m: a DCT-I along y, one
-// tridiagonal solve along x per mode (partition method: block eliminations, cyclic reduction
-// of the blocks' interface system in LDS), and the same DCT-I again (the matrix
-// C[j, m] = cos(pi j m / n) is symmetric).  A'^-1 A has its spectrum in [0.95, 1.003] for
-// eps/h = 2 and closer to 1 as eps/h grows (the mass is a small part of the operator there),
-// so PCG needs 3-5 iterations to 1e-9 whatever the grid.
+// The consistent mass is not such a sum: each of its triangles couples the ends of its cell's
+// diagonal.  Its average over the two ways to draw the diagonals is one, with C = W - T / 2:
+//   M' = (hx hy / 12) [6 W_y (x) W_x + 2 W_y (x) C_x + 2 C_y (x) W_x + 2 C_y (x) C_x],
+// and A' = eps^2 K + M' is diagonalised by the DCT-I in y: T_y v_m = lambda_m W_y v_m with
+// v_m[j] = cos(pi j m / n), lambda_m = 2 - 2 cos(pi m / n), v_m' W_y v_k = D_m delta_mk
+// (D_m = n / 2, or n for m = 0, n).  So A'^-1 r = sum_m v_m (x) X_m^-1 (v_m' r) / D_m with
+//   X_m = (eps^2 hy/hx - hx hy (2 - lambda_m / 2) / 12) T_x
+//         + (eps^2 (hx/hy) lambda_m + hx hy (1 - lambda_m / 6)) W_x,
+// diagonally dominant for any eps: a DCT-I along y, one tridiagonal solve along x per mode
+// (partition method: block eliminations, cyclic reduction of the blocks' interface system in
+// LDS), and the same DCT-I again (the matrix C[j, m] = cos(pi j m / n) is symmetric).  A - A' is
+// the diagonals' antisymmetric part, (hx hy / 6) sin sin in the symbols: with eps/h = 1 the
+// spectrum of A'^-1 A is 1 -+ 0.046, against [0.86, 1] for the lumped mass hx hy W_y (x) W_x
+// (TMX_OPT_FILTER_DCT 1), and both come close to 1 as eps/h grows.  PCG iterations of a filter
+// solve to 1e-11, two solves a step, lumped / averaged:
+// 60 x 20 cells (eps/h = 1) 8 + 8 / 7 + 8, 40 x 40 (0.8) 9 + 9 / 8 + 8, 320 x 160 6 + 6 / 5 + 6,
+// 640 x 320 and above the same.
 //
 // The DCT-I of the n + 1 values of a y-column is computed from a complex FFT of length 2n in
 // LDS (k_dct1_cols): two columns a, b are packed as a + i b and extended evenly
@@ -51,8 +58,9 @@ class DctPrecond {
   // the LDS budget; eps: the filter's length scale
   static bool supported(int nx, int ny, int max_prime);
   int init(int nx, int ny, double hx, double hy, double eps, hipStream_t s);
-  // z = A'^-1 r (vectors of (nx + 1)(ny + 1) values), partials of r.z into rz if given
-  int apply(const T* r, T* z, RedSlot* rz, hipStream_t s);
+  // z = A'^-1 r (vectors of (nx + 1)(ny + 1) values; lumped: with the lumped mass in A'),
+  // partials of r.z into rz if given
+  int apply(const T* r, T* z, bool lumped, RedSlot* rz, hipStream_t s);
 
   // Largest prime factor p of 2 ny: a prime without a butterfly costs p products per point
   // (fft_stage_direct), the V-cycle the same per point whatever ny.  One filter solve to 1e-11,

@@ -414,8 +414,8 @@ static size_t dct_tri_lds(int mx) {
 }
 
 template <typename T>
-__device__ __forceinline__ void dct_tri_body(const BlkId blk, int mx, int n, T a_off,
-                                             double hxhy, double cy, T* modes_) {
+__device__ __forceinline__ void dct_tri_body(const BlkId blk, int mx, int n, double a0,
+                                             double hxhy, double cy, int lumped, T* modes_) {
   const auto modes = glob(modes_);
   extern __shared__ __align__(16) unsigned char tri_lds[];
   const int k = (mx + kTriThreads - 1) / kTriThreads;
@@ -430,7 +430,10 @@ __device__ __forceinline__ void dct_tri_body(const BlkId blk, int mx, int n, T a
   const int mode = (int)blk.id;
   T* row = modes + (size_t)mode * mx;
   const double lam = 2.0 - 2.0 * std::cos(M_PI * (double)mode / (double)n);
-  const T c = (T)(hxhy + cy * lam);
+  // (a0 - hxhy (2 - lam / 2) / 12) T_x + (cy lam + hxhy (1 - lam / 6)) W_x, or a0 T_x +
+  // (cy lam + hxhy) W_x with the lumped mass
+  const T a_off = (T)(lumped ? a0 : a0 - hxhy * (2.0 - 0.5 * lam) / 12.0);
+  const T c = (T)(cy * lam + (lumped ? hxhy : hxhy * (1.0 - lam / 6.0)));
   const T inv_d = (mode == 0 || mode == n) ? T(1) / (T)n : T(2) / (T)n;
   const T b_in = a_off * T(2) + c, b_edge = a_off + c * T(0.5);
   const int tid = threadIdx.x;
@@ -544,9 +547,10 @@ __device__ __forceinline__ void dct_tri_body(const BlkId blk, int mx, int n, T a
 }
 
 template <typename T>
-__global__ __launch_bounds__(kTriThreads) void k_dct_tri(int mx, int n, T a_off, double hxhy,
-                                                         double cy, T* __restrict__ modes) {
-  dct_tri_body<T>(hw_blk(), mx, n, a_off, hxhy, cy, modes);
+__global__ __launch_bounds__(kTriThreads) void k_dct_tri(int mx, int n, double a0, double hxhy,
+                                                         double cy, int lumped,
+                                                         T* __restrict__ modes) {
+  dct_tri_body<T>(hw_blk(), mx, n, a0, hxhy, cy, lumped, modes);
 }
 
 // LDS of k_dct1_cols: the complex sequences of `cols` columns (2 n points each per pair) and
@@ -627,7 +631,7 @@ int DctPrecond<T>::init(int nx, int ny, double hx, double hy, double eps, hipStr
 }
 
 template <typename T>
-int DctPrecond<T>::apply(const T* r, T* z, RedSlot* rz, hipStream_t s) {
+int DctPrecond<T>::apply(const T* r, T* z, bool lumped, RedSlot* rz, hipStream_t s) {
   const int n = ny_, mx = mx_;
   const int cols = dct_cols<T>(n);
   const int groups = (mx + cols - 1) / cols;
@@ -640,9 +644,9 @@ int DctPrecond<T>::apply(const T* r, T* z, RedSlot* rz, hipStream_t s) {
                              static_cast<const T*>(nullptr), static_cast<double*>(nullptr));
   TMX_HIP(hipGetLastError());
   // tridiagonal solves along x, one workgroup per mode (scaled by 1 / D_m there)
-  const T a_off = (T)(eps_ * eps_ * hy_ / hx_);
+  const double a0 = eps_ * eps_ * hy_ / hx_;
   const double cy = eps_ * eps_ * hx_ / hy_;
-  TMX_LAUNCH_OR_RECORD(kTriThreads, (dct_tri_body<T>), n + 1, dct_tri_lds<T>(mx), s, (k_dct_tri<T>), mx, n, a_off, hx_ * hy_, cy, t);
+  TMX_LAUNCH_OR_RECORD(kTriThreads, (dct_tri_body<T>), n + 1, dct_tri_lds<T>(mx), s, (k_dct_tri<T>), mx, n, a0, hx_ * hy_, cy, lumped ? 1 : 0, t);
   TMX_HIP(hipGetLastError());
   // inverse: z[j] = sum_m t[m] cos(pi j m / n), with the partials of r.z
   double* part = nullptr;

@@ -743,7 +743,7 @@ int Hierarchy::vcycle(int l, const T* b, T* out, hipStream_t s, RedSlot* dot_bz)
       TMX_TRY(d->init(levels_[0].nx, levels_[0].ny, levels_[0].hx, levels_[0].hy, eps_, s));
       dct = std::move(d);
     }
-    return dct->apply(b, out, dot_bz, s);
+    return dct->apply(b, out, use_dct_ == 1, dot_bz, s);
   }
   Level& L = levels_[l];
   Level& C = levels_[l + 1];
