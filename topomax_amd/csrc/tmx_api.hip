@@ -1048,6 +1048,7 @@ extern "C" int tmx_bench_kernel(tmx_problem* h, int kernel, int precision, int r
     }
     if (kernel >= 3) {  // paired sweeps with the handle's chunk heights
       const int op1 = kernel == 3 ? kSmoothZero : kProlongSmooth;
+      if (kernel != 3 && !h->el.pair_post_ok()) return invalid("kernel 4 needs even nx and ny");
       const int rows = (kernel == 3 ? h->el.pair_rows_ : h->el.pair_rows_post_)[f64 ? 1 : 0];
       if (f64)
         return h->el.sweep_pair0<double>(op1, rows, h->u_s.get(), h->Fm.get(), h->tmp64.get(),

@@ -90,16 +90,19 @@ hipError_t elast_sweep(const ElastOpArgs<T>& a, int op, const T* x, const T* b, 
 
 // Two block-Jacobi sweeps in one launch: op1 = kSmoothZero (y = S2 S1 0) or kProlongSmooth
 // (y = S2 S1 (x + P ec)), with damping om1, om2 and node-row chunks of `rows`; a dot slot
-// receives partials of b.y.  Same results as the two launches up to round-off.
+// receives partials of b.y.  Same results as the two launches up to round-off.  bilinear: P of
+// a tensor-product coarse grid (prolong_bilinear) instead of the nested one.
 template <typename T>
 hipError_t elast_sweep_pair(const ElastOpArgs<T>& a, int op1, int rows, const T* x, const T* b,
-                            T* y, T om1, T om2, RedSlot* dot, hipStream_t s, const T* ec);
+                            T* y, T om1, T om2, RedSlot* dot, hipStream_t s, const T* ec,
+                            bool bilinear = false);
 
 // The zero-start pair (y = S2 S1 0) with the residual b - A y restricted to the nested coarse
 // grid in the same launch (yc); nx, ny even, node-row chunks of `rows` (rounded down to even).
+// bilinear: restricted to a tensor-product coarse grid (restrict_bilinear); any nx, ny.
 template <typename T>
 hipError_t elast_sweep_pair_rr(const ElastOpArgs<T>& a, int rows, const T* b, T* y, T* yc,
-                               T om1, T om2, hipStream_t s);
+                               T om1, T om2, hipStream_t s, bool bilinear = false);
 
 // per-cell mean r from nodal xi (for restriction of level-0 weights); with cellw32, also
 // their FP32 copy

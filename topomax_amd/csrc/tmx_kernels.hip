@@ -122,6 +122,7 @@ struct RowIn {
   V2<T> w = {T(0), T(0)};
   V2<T> b = {T(0), T(0)};
   V2<T> x = {T(0), T(0)}, e = {T(0), T(0)}, e1 = {T(0), T(0)};  // iterate, coarse correction
+  V2<T> e2 = {T(0), T(0)}, e3 = {T(0), T(0)};
 };
 
 template <typename T, bool XI, int OP>
@@ -402,7 +403,9 @@ template hipError_t elast_sweep<float>(const ElastOpArgs<float>&, int, const flo
 // completes its node row cy; the second sweep then takes cell row cy - 1 between the first
 // sweep's node rows cy - 1 and cy and completes its node row cy - 1.  A chunk of R node rows
 // sweeps R + 3 cell rows (node rows r0 - 1 .. rend of the first sweep).
-template <typename T, bool XI, int OP1>
+// BIL: P is the tensor-product interpolation of a coarse grid with ceil(n / 2) cells per axis
+// (odd grids) instead of the nested one.
+template <typename T, bool XI, int OP1, bool BIL>
 __device__ __forceinline__ void elast_sweep_pair_body(const BlkId blk, const ElastOpArgs<T>& a,
                                                       const T* x, const T* b, T* y, T om1, T om2,
                                                       double* dpart, const T* ec) {
@@ -416,7 +419,7 @@ __device__ __forceinline__ void elast_sweep_pair_body(const BlkId blk, const Ela
   const int strip = wv % sh.nstrips, chunk = wv / sh.nstrips;
   const bool wave_ok = chunk < sh.nchunks;
   const int nx = sh.nx, ny = sh.ny, nvx = nx + 1;
-  const int nxc = nx >> 1;
+  const int nxc = BIL ? (nx + 1) >> 1 : nx >> 1;
   const int c = strip * sh.stripw - H + lane;
   const bool colv = wave_ok && c >= 0 && c <= nx;
   const bool cellc = wave_ok && c >= 0 && c < nx;
@@ -440,23 +443,6 @@ __device__ __forceinline__ void elast_sweep_pair_body(const BlkId blk, const Ela
   auto row_fixed = [&](int iy) {
     return colfix || ((fixed & kBottom) && iy == 0) || ((fixed & kTop) && iy == ny);
   };
-  auto ld_x = [&](int iy, V& raw) -> V {  // x + P e (kProlongSmooth)
-    V v = zero;
-    const bool ok = colv && iy >= 0 && iy <= ny;
-    if (ok) v = X[(unsigned)(iy * nvx + c)];
-    if (ok && !row_fixed(iy)) {
-      const int I0 = c >> 1, J0 = iy >> 1, ox = c & 1, oy = iy & 1;
-      V e = EC[(size_t)J0 * (nxc + 1) + I0];
-      if (ox | oy) {
-        const V e1 = EC[(size_t)(J0 + oy) * (nxc + 1) + I0 + ox];
-        e = {T(0.5) * (e.x + e1.x), T(0.5) * (e.y + e1.y)};
-      }
-      v += e;
-    }
-    raw = v;
-    if (row_fixed(iy)) v = zero;
-    return v;
-  };
   auto ld_xi = [&](int iy) -> T {
     if (XI && colv && iy >= 0 && iy <= ny) return XIP[(unsigned)(iy * nvx + c)];
     return T(0);
@@ -465,10 +451,6 @@ __device__ __forceinline__ void elast_sweep_pair_body(const BlkId blk, const Ela
   int cy = cy_begin;
   // first sweep: cell row cy between node rows cy (u_b) and cy + 1
   V ub = zero, ub_raw = zero, ubr = zero;
-  if constexpr (PS) {
-    ub = ld_x(cy, ub_raw);
-    ubr = lane_down(ub);
-  }
   T zb = ld_xi(cy);
   T zbr = lane_down(zb);
   V acc1 = zero;                            // forces on node row cy from cell row cy - 1
@@ -487,6 +469,9 @@ __device__ __forceinline__ void elast_sweep_pair_body(const BlkId blk, const Ela
   // nodes and the interpolation are applied at the row's turn (see k_elast_sweep_pair_rr)
   const int cn = min(max(c, 0), nx), cc = min(max(c, 0), nx - 1);
   const int I0 = cn >> 1, ox = cn & 1;
+  // the column's interpolation weights: an even node lies on coarse node c / 2, the last one of
+  // an odd count on the last coarse node, any other odd node half way
+  const T bx1 = ox ? (cn == nx ? T(1) : T(0.5)) : T(0), bx0 = T(1) - bx1;
   auto fetch = [&](int row) {
     RowIn<T> r;
     const int nt = min(max(row + 1, 0), ny), nb = min(max(row, 0), ny);
@@ -496,26 +481,41 @@ __device__ __forceinline__ void elast_sweep_pair_body(const BlkId blk, const Ela
       r.x = X[(unsigned)(nt * nvx + cn)];
       r.e = EC[(size_t)J0 * (nxc + 1) + I0];
       r.e1 = EC[(size_t)(J0 + oy) * (nxc + 1) + I0 + ox];
+      if constexpr (BIL) {  // (an even node's second neighbour is itself, with weight zero)
+        r.e2 = EC[(size_t)J0 * (nxc + 1) + I0 + ox];
+        r.e3 = EC[(size_t)(J0 + oy) * (nxc + 1) + I0];
+      }
     }
     if constexpr (XI) r.z = XIP[(unsigned)(nt * nvx + cn)];
     else r.w = CW[(unsigned)(cr * nx + cc)];
     r.b = B[(unsigned)(nb * nvx + cn)];
     return r;
   };
-  // x + P e at node row iy from its prefetched values (as ld_x)
+  // x + P e at node row iy from its prefetched values (raw: before fixed nodes are zeroed)
   auto form_x = [&](int iy, const RowIn<T>& in, V& raw) -> V {
     V v = zero;
     const bool ok = colv && iy >= 0 && iy <= ny;
     if (ok) v = in.x;
     if (ok && !row_fixed(iy)) {
       V e = in.e;
-      if (ox | (iy & 1)) e = {T(0.5) * (e.x + in.e1.x), T(0.5) * (e.y + in.e1.y)};
+      if constexpr (BIL) {
+        const T y1 = (iy & 1) ? (iy == ny ? T(1) : T(0.5)) : T(0), y0 = T(1) - y1;
+        const T a00 = bx0 * y0, a10 = bx1 * y0, a01 = bx0 * y1, a11 = bx1 * y1;
+        e = {a00 * in.e.x + a10 * in.e2.x + a01 * in.e3.x + a11 * in.e1.x,
+             a00 * in.e.y + a10 * in.e2.y + a01 * in.e3.y + a11 * in.e1.y};
+      } else if (ox | (iy & 1)) {
+        e = {T(0.5) * (e.x + in.e1.x), T(0.5) * (e.y + in.e1.y)};
+      }
       v += e;
     }
     raw = v;
     if (row_fixed(iy)) v = zero;
     return v;
   };
+  if constexpr (PS) {
+    if (wave_ok) ub = form_x(cy, fetch(cy - 1), ub_raw);
+    ubr = lane_down(ub);
+  }
   RowIn<T> pf[kPrefetchRows];
   if (wave_ok) {
 #pragma unroll
@@ -632,21 +632,22 @@ __device__ __forceinline__ void elast_sweep_pair_body(const BlkId blk, const Ela
   }
 }
 
-template <typename T, bool XI, int OP1>
+template <typename T, bool XI, int OP1, bool BIL>
 __global__ __launch_bounds__(kBlock) void k_elast_sweep_pair(ElastOpArgs<T> a,
                                                              const T* __restrict__ x,
                                                              const T* __restrict__ b,
                                                              T* __restrict__ y, T om1, T om2,
                                                              double* __restrict__ dpart,
                                                              const T* __restrict__ ec) {
-  elast_sweep_pair_body<T, XI, OP1>(hw_blk(), a, x, b, y, om1, om2, dpart, ec);
+  elast_sweep_pair_body<T, XI, OP1, BIL>(hw_blk(), a, x, b, y, om1, om2, dpart, ec);
 }
 
 template <typename T>
 hipError_t elast_sweep_pair(const ElastOpArgs<T>& a0, int op1, int rows, const T* x, const T* b,
-                            T* y, T om1, T om2, RedSlot* dot_by, hipStream_t s, const T* ec) {
+                            T* y, T om1, T om2, RedSlot* dot_by, hipStream_t s, const T* ec,
+                            bool bilinear) {
   if (op1 != kSmoothZero && op1 != kProlongSmooth) return hipErrorInvalidValue;
-  if (op1 == kProlongSmooth && (!ec || !x || (a0.sh.nx & 1) || (a0.sh.ny & 1)))
+  if (op1 == kProlongSmooth && (!ec || !x || (!bilinear && ((a0.sh.nx & 1) || (a0.sh.ny & 1)))))
     return hipErrorInvalidValue;
   if (!b || !y || (!a0.xi && !a0.cellw)) return hipErrorInvalidValue;
   if ((size_t)(a0.sh.nx + 1) * (a0.sh.ny + 1) >= (1ull << 31)) return hipErrorInvalidValue;
@@ -660,25 +661,28 @@ hipError_t elast_sweep_pair(const ElastOpArgs<T>& a0, int op1, int rows, const T
     dot_by->nblocks = nb;
   }
   const bool xi = a.xi != nullptr;
-#define TMX_LAUNCH(XIV, OPV)                                                              \
-  TMX_LAUNCH_OR_RECORD(kBlock, (elast_sweep_pair_body<T, XIV, OPV>), nb, 0, s,              \
-                       (k_elast_sweep_pair<T, XIV, OPV>), a, x, b, y, om1, om2, dp, ec)
+#define TMX_LAUNCH(XIV, OPV, BILV)                                                        \
+  TMX_LAUNCH_OR_RECORD(kBlock, (elast_sweep_pair_body<T, XIV, OPV, BILV>), nb, 0, s,        \
+                       (k_elast_sweep_pair<T, XIV, OPV, BILV>), a, x, b, y, om1, om2, dp, ec)
   if (op1 == kSmoothZero) {
-    if (xi) TMX_LAUNCH(true, kSmoothZero);
-    else TMX_LAUNCH(false, kSmoothZero);
+    if (xi) TMX_LAUNCH(true, kSmoothZero, false);
+    else TMX_LAUNCH(false, kSmoothZero, false);
+  } else if (bilinear) {
+    if (xi) TMX_LAUNCH(true, kProlongSmooth, true);
+    else TMX_LAUNCH(false, kProlongSmooth, true);
   } else {
-    if (xi) TMX_LAUNCH(true, kProlongSmooth);
-    else TMX_LAUNCH(false, kProlongSmooth);
+    if (xi) TMX_LAUNCH(true, kProlongSmooth, false);
+    else TMX_LAUNCH(false, kProlongSmooth, false);
   }
 #undef TMX_LAUNCH
   return hipGetLastError();
 }
 template hipError_t elast_sweep_pair<double>(const ElastOpArgs<double>&, int, int, const double*,
                                              const double*, double*, double, double, RedSlot*,
-                                             hipStream_t, const double*);
+                                             hipStream_t, const double*, bool);
 template hipError_t elast_sweep_pair<float>(const ElastOpArgs<float>&, int, int, const float*,
                                             const float*, float*, float, float, RedSlot*,
-                                            hipStream_t, const float*);
+                                            hipStream_t, const float*, bool);
 
 // The zero-start pair with the residual and its nested restriction fused behind it: three
 // stages, each trailing the one before by a cell row.  At cell row cy the first sweep completes
@@ -688,7 +692,14 @@ template hipError_t elast_sweep_pair<float>(const ElastOpArgs<float>&, int, int,
 // cy - 2; once the residual rows 2J - 1 .. 2J + 1 exist, the lanes of even columns write
 // coarse node row J.  The lanes carry four halo columns on each side (56 output columns); a
 // chunk of R (even) node rows sweeps R + 6 cell rows.
-template <typename T, bool XI>
+// BIL: the restriction is the transpose of the tensor-product interpolation from a coarse grid
+// with ceil(n / 2) cells per axis (odd grids): coarse node (I, J) lies on fine node min(2I, nx),
+// min(2J, ny), and takes half of each neighbour that lies half way, per axis; the sum is kept
+// in double, as in the separate restriction.  Against separate residual, restriction and
+// prolongation launches (and elast_sweep_pair BIL) a whole step takes, in us, FP64 333 x 111
+// cells 2150 -> 2045, 999 x 333 4288 -> 4180, 2991 x 997 25753 -> 24418; mixed 1971 -> 1839,
+// 3981 -> 3891, 21318 -> 20274.
+template <typename T, bool XI, bool BIL>
 __device__ __forceinline__ void elast_sweep_pair_rr_body(const BlkId blk, const ElastOpArgs<T>& a,
                                                          const T* b, T* y, T* yc, T om1, T om2) {
   using V = V2<T>;
@@ -699,7 +710,7 @@ __device__ __forceinline__ void elast_sweep_pair_rr_body(const BlkId blk, const 
   const int strip = wv % sh.nstrips, chunk = wv / sh.nstrips;
   const bool wave_ok = chunk < sh.nchunks;
   const int nx = sh.nx, ny = sh.ny, nvx = nx + 1;
-  const int nxc = nx >> 1, nyc = ny >> 1;
+  const int nxc = BIL ? (nx + 1) >> 1 : nx >> 1, nyc = BIL ? (ny + 1) >> 1 : ny >> 1;
   const int c = strip * sh.stripw - H + lane;
   const bool colv = wave_ok && c >= 0 && c <= nx;
   const bool cellc = wave_ok && c >= 0 && c < nx;
@@ -854,7 +865,31 @@ __device__ __forceinline__ void elast_sweep_pair_rr_body(const BlkId blk, const 
     // coarse row J: centre fine row 2J = rk - 1 (rk odd), or 2J = ny at the top (ny even)
     const bool odd_emit = (rk & 1) && rk - 1 >= r0 && rk - 1 < rend;
     const bool top_emit = rk == ny && ny >= r0 && ny < rend;
-    if (odd_emit || top_emit) {
+    if constexpr (BIL) {
+      // (the values beyond the grid are zero)
+      const double wl = (c & 1) ? 0.0 : 0.5;
+      const double wr = (c & 1) || ((nx & 1) && c + 1 == nx) ? 0.0 : 0.5;
+      auto emit = [&](int J, V lo, V mid, V hi) {
+        const V ll = lane_up(lo), lr = lane_down(lo), ml = lane_up(mid), mr = lane_down(mid);
+        const V hl = lane_up(hi), hr = lane_down(hi);
+        if (outl && (!(c & 1) || c == nx)) {
+          const int I = (c + 1) >> 1;
+          double ox = 0.0, oy = 0.0;
+          if (!node_fixed(fixed, I, J, nxc, nyc)) {
+            ox = ((double)mid.x + wl * (double)ml.x + wr * (double)mr.x) +
+                 0.5 * (((double)lo.x + wl * (double)ll.x + wr * (double)lr.x) +
+                        ((double)hi.x + wl * (double)hl.x + wr * (double)hr.x));
+            oy = ((double)mid.y + wl * (double)ml.y + wr * (double)mr.y) +
+                 0.5 * (((double)lo.y + wl * (double)ll.y + wr * (double)lr.y) +
+                        ((double)hi.y + wl * (double)hl.y + wr * (double)hr.y));
+          }
+          YC[(size_t)J * (nxc + 1) + I] = {(T)ox, (T)oy};
+        }
+      };
+      const bool last_odd = (ny & 1) && rk == ny;  // (row ny belongs to the last coarse row alone)
+      if (odd_emit) emit((rk - 1) >> 1, rA, rB, last_odd ? zero : rC);
+      if (top_emit) emit(nyc, last_odd ? zero : rB, rC, zero);
+    } else if (odd_emit || top_emit) {
       const V lo = odd_emit ? rA : rB, mid = odd_emit ? rB : rC;
       const V hi = odd_emit ? rC : zero;
       const V mr = lane_down(mid), ml = lane_up(mid), hr = lane_down(hi), ll = lane_up(lo);
@@ -894,36 +929,42 @@ __device__ __forceinline__ void elast_sweep_pair_rr_body(const BlkId blk, const 
   }
 }
 
-template <typename T, bool XI>
+template <typename T, bool XI, bool BIL>
 __global__ __launch_bounds__(kBlock) void k_elast_sweep_pair_rr(ElastOpArgs<T> a,
                                                                 const T* __restrict__ b,
                                                                 T* __restrict__ y,
                                                                 T* __restrict__ yc, T om1,
                                                                 T om2) {
-  elast_sweep_pair_rr_body<T, XI>(hw_blk(), a, b, y, yc, om1, om2);
+  elast_sweep_pair_rr_body<T, XI, BIL>(hw_blk(), a, b, y, yc, om1, om2);
 }
 
 template <typename T>
 hipError_t elast_sweep_pair_rr(const ElastOpArgs<T>& a0, int rows, const T* b, T* y, T* yc,
-                               T om1, T om2, hipStream_t s) {
+                               T om1, T om2, hipStream_t s, bool bilinear) {
   if (!b || !y || !yc || (!a0.xi && !a0.cellw)) return hipErrorInvalidValue;
-  if ((a0.sh.nx & 1) || (a0.sh.ny & 1)) return hipErrorInvalidValue;
+  if (!bilinear && ((a0.sh.nx & 1) || (a0.sh.ny & 1))) return hipErrorInvalidValue;
   if ((size_t)(a0.sh.nx + 1) * (a0.sh.ny + 1) >= (1ull << 31)) return hipErrorInvalidValue;
   ElastOpArgs<T> a = a0;
   a.sh = SweepShape::make(a0.sh.nx, a0.sh.ny, std::max(2, rows & ~1), kWave - 2 * 4);
   const int nb = a.sh.blocks();
-  if (a.xi)
-    TMX_LAUNCH_OR_RECORD(kBlock, (elast_sweep_pair_rr_body<T, true>), nb, 0, s,
-                         (k_elast_sweep_pair_rr<T, true>), a, b, y, yc, om1, om2);
-  else
-    TMX_LAUNCH_OR_RECORD(kBlock, (elast_sweep_pair_rr_body<T, false>), nb, 0, s,
-                         (k_elast_sweep_pair_rr<T, false>), a, b, y, yc, om1, om2);
+#define TMX_LAUNCH(XIV, BILV)                                                             \
+  TMX_LAUNCH_OR_RECORD(kBlock, (elast_sweep_pair_rr_body<T, XIV, BILV>), nb, 0, s,          \
+                       (k_elast_sweep_pair_rr<T, XIV, BILV>), a, b, y, yc, om1, om2)
+  if (bilinear) {
+    if (a.xi) TMX_LAUNCH(true, true);
+    else TMX_LAUNCH(false, true);
+  } else {
+    if (a.xi) TMX_LAUNCH(true, false);
+    else TMX_LAUNCH(false, false);
+  }
+#undef TMX_LAUNCH
   return hipGetLastError();
 }
 template hipError_t elast_sweep_pair_rr<double>(const ElastOpArgs<double>&, int, const double*,
-                                                double*, double*, double, double, hipStream_t);
+                                                double*, double*, double, double, hipStream_t,
+                                                bool);
 template hipError_t elast_sweep_pair_rr<float>(const ElastOpArgs<float>&, int, const float*,
-                                               float*, float*, float, float, hipStream_t);
+                                               float*, float*, float, float, hipStream_t, bool);
 
 template <typename T>
 __device__ __forceinline__ void elast_cell_weights_body(const BlkId blk, int nx,

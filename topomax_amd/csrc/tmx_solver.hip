@@ -551,16 +551,18 @@ int Hierarchy::sweep_pair0(int op1, int rows, const T* x, const T* b, T* y, doub
     return -1;
   }
   const T* ec = nullptr;
+  bool bilinear = false;
   if (op1 == kProlongSmooth) {
-    if (!pair_post_ok(l)) {
-      set_error("internal: paired prolongation needs a nested level below");
+    if (l + 1 >= (int)levels_.size()) {
+      set_error("internal: paired prolongation needs a level below");
       return -1;
     }
+    bilinear = !levels_[l + 1].nested_from_prev;
     ec = PrecBufs<T>::x(levels_[l + 1]);
   }
   const ElastOpArgs<T> a = elast_args<T>(*this, l, xi_for<T>(*this), PrecBufs<T>::cw(levels_[l]),
                                          sizeof(T) == 8, true);
-  TMX_HIP(elast_sweep_pair<T>(a, op1, rows, x, b, y, (T)om1, (T)om2, dot, s, ec));
+  TMX_HIP(elast_sweep_pair<T>(a, op1, rows, x, b, y, (T)om1, (T)om2, dot, s, ec, bilinear));
   return 0;
 }
 
@@ -592,14 +594,15 @@ int Hierarchy::filter_pipe0(bool down, int rows, hipStream_t s) {
 template <typename T>
 int Hierarchy::sweep_pair_rr0(int rows, const T* b, T* y, double om1, double om2, hipStream_t s,
                               int l) {
-  if (phys_ != kElasticity || !pair_post_ok(l) || levels_[l].kind != kElem || rows < 1) {
-    set_error("internal: fused restriction needs an elasticity element level over a nested one");
+  if (phys_ != kElasticity || l < 0 || l + 1 >= (int)levels_.size() ||
+      levels_[l].kind != kElem || rows < 1) {
+    set_error("internal: fused restriction needs an elasticity element level over another");
     return -1;
   }
   const ElastOpArgs<T> a = elast_args<T>(*this, l, xi_for<T>(*this), PrecBufs<T>::cw(levels_[l]),
                                          sizeof(T) == 8, true);
   TMX_HIP(elast_sweep_pair_rr<T>(a, rows, b, y, PrecBufs<T>::b(levels_[l + 1]), (T)om1, (T)om2,
-                                 s));
+                                 s, !levels_[l + 1].nested_from_prev));
   return 0;
 }
 
@@ -793,8 +796,9 @@ int Hierarchy::vcycle(int l, const T* b, T* out, hipStream_t s, RedSlot* dot_bz)
   const int rows_post = l == 0 ? pair_rows_post_[pi] : pair_rows_coarse_[1];
   const int rows_rr = l == 0 ? pair_rr_rows_[pi] : pair_rows_coarse_[2];
   const bool pair_pre = pair_level && rows_pre > 0 && npre >= 2;
-  const bool pair_post = pair_level && rows_post > 0 && fused_el && npost >= 2;
-  const bool pair_rr = pair_pre && npre == 2 && fused_el && rows_rr > 0;
+  const bool pair_fused = fused_ && pair_level;  // (nested or bilinear transfers)
+  const bool pair_post = pair_fused && rows_post > 0 && npost >= 2;
+  const bool pair_rr = pair_pre && npre == 2 && pair_fused && rows_rr > 0;
   const int launches = npre - (pair_pre ? 1 : 0) + npost - (pair_post ? 1 : 0);
   int w = (launches - 1) % 2;
   int kpre = 1;
