@@ -34,6 +34,8 @@ constexpr int kBandThreadsWide = 1024;
 // workgroup size of the mid variant (option): the same tiles as kBandThreads, twice the threads
 constexpr int kBandThreadsMid = 512;
 constexpr size_t kBandLdsBytes = 64 * 1024;
+// fewest workgroups for which a 9-point level takes the 16 x 12 tiles of the mid variant
+constexpr int kBandMidTiles = 100;
 
 // where a level's operator comes from
 enum BandSrc : int {
@@ -58,7 +60,8 @@ struct BandLevel {
   T omega_down[kMaxNu];  // step size of each sweep
   T omega_up[kMaxNu];
   int tx, ty;            // owned fine tile (nodes), even
-  int wide;              // 1: kSrcCells levels may use the kBandThreadsWide variant;
+  int wide;              // 2 with kSrcStencil: kBandThreadsMid threads, if one node each;
+                         // 1: kSrcCells levels may use the kBandThreadsWide variant;
                          // 2 / 3: kSrcCells levels run kBandThreadsMid / kBandThreadsWide
                          // threads on the standard tiles
 };

@@ -732,7 +732,9 @@ hipError_t band_down(const BandLevel<T>& L, const T* b, T* x, T* bc, hipStream_t
   } else if (L.wide == 1 && L.src == kSrcCells && !one && ne <= (size_t)kBandThreadsWide) {
     launch_down<T, BS, kSrcCells, true, kBandThreadsWide>(L, b, x, bc, lds, s);
   } else if (L.src == kSrcStencil) {
-    if (one) launch_down<T, BS, kSrcStencil, true>(L, b, x, bc, lds, s);
+    if (L.wide == 2 && ne <= (size_t)kBandThreadsMid)
+      launch_down<T, BS, kSrcStencil, true, kBandThreadsMid>(L, b, x, bc, lds, s);
+    else if (one) launch_down<T, BS, kSrcStencil, true>(L, b, x, bc, lds, s);
     else launch_down<T, BS, kSrcStencil, false>(L, b, x, bc, lds, s);
   } else if (L.src == kSrcCells) {
     if (one) launch_down<T, BS, kSrcCells, true>(L, b, x, bc, lds, s);
@@ -773,7 +775,9 @@ hipError_t band_up(const BandLevel<T>& L, const T* x, const T* ec, const T* b, T
              !part) {
     launch_up<T, BS, kSrcCells, true, kBandThreadsWide>(L, x, ec, b, y, part, lds, s);
   } else if (L.src == kSrcStencil) {
-    if (one) launch_up<T, BS, kSrcStencil, true>(L, x, ec, b, y, part, lds, s);
+    if (L.wide == 2 && ne <= (size_t)kBandThreadsMid && !part)
+      launch_up<T, BS, kSrcStencil, true, kBandThreadsMid>(L, x, ec, b, y, part, lds, s);
+    else if (one) launch_up<T, BS, kSrcStencil, true>(L, x, ec, b, y, part, lds, s);
     else launch_up<T, BS, kSrcStencil, false>(L, x, ec, b, y, part, lds, s);
   } else if (L.src == kSrcCells) {
     if (one) launch_up<T, BS, kSrcCells, true>(L, x, ec, b, y, part, lds, s);

@@ -711,6 +711,27 @@ static bool band_level(const Hierarchy& h, int l, BandLevel<T>& B) {
       return true;
     }
   }
+  if (h.band_wide_ == 2 && l > 0 && B.src == kSrcStencil) {
+    // A 9-point level whose 16 x 12 tiles make kBandMidTiles workgroups or more: with a halo for
+    // three sweeps such a tile is 24 x 20 nodes, one per thread of kBandThreadsMid, so the rows
+    // (36 values a node, by far the most of the launch's bytes) are read once and stay in
+    // registers, where the tiles below read them again for every sweep (16 x 8 and larger) or
+    // read four rows per owned node (8 x 8 in 256 threads).  Whole steps at rtol 1e-10 in us,
+    // those tiles -> these: FP64 801 x 267 cells 4985 -> 4778, 999 x 333 4141 -> 3772,
+    // 1203 x 401 9071 -> 8006, 1731 x 577 18586 -> 17645; mixed 4238 -> 4136, 3913 -> 3666,
+    // 7227 -> 6461, 15928 -> 13741.  With fewer workgroups the chip is less full than with
+    // 8 x 8 tiles: 78 (399 x 133 cells, FP64) 2451 -> 2473, 45 (201 x 67 and 333 x 111 below
+    // level 1) 2060 -> 2072; 105 (450 x 151) 2760 -> 2702.
+    const int nu = std::max(B.nu_down, B.nu_up);
+    if (band_ext(16, nu, true) * band_ext(12, nu, true) <= (size_t)kBandThreadsMid &&
+        band_lds_bytes(16, 12, nu, h.bs_, sizeof(T), B.src, true) <= kBandLdsBytes &&
+        band_tiles(L.nx, L.ny, 16, 12) >= kBandMidTiles) {
+      B.tx = 16;
+      B.ty = 12;
+      B.wide = 2;
+      return true;
+    }
+  }
   static const int cand[][2] = {{32, 32}, {32, 16}, {16, 16}, {16, 8}, {8, 8}};
   bool found = false;
   for (const auto& c : cand) {
