@@ -254,7 +254,8 @@ enum tmx_option {
                                    workgroups; 1: 1024 threads with one node per thread (square
                                    tiles, e.g. 24 x 24), each node's row built once per launch;
                                    2 (default): 512 threads on the standard tiles, and on
-                                   16 x 12 tiles of large 9-point levels; 3: 1024 */
+                                   16 x 12 tiles of larger levels, 9-point ones too;
+                                   3: 1024 */
   TMX_OPT_BENCH_COLD = 26,      /* 1: tmx_bench_kernel times each launch alone after reading
                                    512 MiB (no inputs left in the caches); 0: back to back */
   TMX_OPT_RU_EVERY = 27,        /* TMX_MIXED_RU: iterations between residual replacements

@@ -1,5 +1,5 @@
-"""9-point levels on the 512-thread tiles of the band kernels (one node per thread, rows kept in
-registers) against the launch-per-sweep V-cycle: the same sweeps in the same order, so the
+"""Levels on the 512-thread 16 x 12 tiles of the band kernels (one node per thread, rows kept in
+registers), 9-point and cell-weight ones, against the launch-per-sweep V-cycle: the same sweeps in the same order, so the
 preconditioner output agrees to round-off, 1e-12 relative in FP64 and 1e-5 in FP32.
 
 Level 1 of these grids has from just below to far above the number of 16 x 12 tiles from which
@@ -15,7 +15,9 @@ pytestmark = pytest.mark.gpu
 
 # level 1 of a x b cells: tiles of 16 x 12 nodes
 SHAPES = [(351, 191), (319, 238), (321, 241), (511, 255), (512, 257), (513, 256), (1, 2399),
-          (2, 2401), (3201, 3), (450, 151)]
+          (2, 2401), (3201, 3), (450, 151),
+          # level 1 with cell weights: 90, 105, 512, 646 and 1066 tiles, and beside them
+          (288, 238), (448, 166), (1022, 382), (1200, 400), (1602, 494)]
 
 
 def rel(a, b):

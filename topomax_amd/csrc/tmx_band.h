@@ -34,7 +34,7 @@ constexpr int kBandThreadsWide = 1024;
 // workgroup size of the mid variant (option): the same tiles as kBandThreads, twice the threads
 constexpr int kBandThreadsMid = 512;
 constexpr size_t kBandLdsBytes = 64 * 1024;
-// fewest workgroups for which a 9-point level takes the 16 x 12 tiles of the mid variant
+// fewest workgroups for which a level takes the 16 x 12 tiles of the mid variant
 constexpr int kBandMidTiles = 100;
 
 // where a level's operator comes from

@@ -711,7 +711,7 @@ static bool band_level(const Hierarchy& h, int l, BandLevel<T>& B) {
       return true;
     }
   }
-  if (h.band_wide_ == 2 && l > 0 && B.src == kSrcStencil) {
+  if (h.band_wide_ == 2 && l > 0 && B.src != kSrcUnit) {
     // A 9-point level whose 16 x 12 tiles make kBandMidTiles workgroups or more: with a halo for
     // three sweeps such a tile is 24 x 20 nodes, one per thread of kBandThreadsMid, so the rows
     // (36 values a node, by far the most of the launch's bytes) are read once and stay in
@@ -722,10 +722,17 @@ static bool band_level(const Hierarchy& h, int l, BandLevel<T>& B) {
     // 7227 -> 6461, 15928 -> 13741.  With fewer workgroups the chip is less full than with
     // 8 x 8 tiles: 78 (399 x 133 cells, FP64) 2451 -> 2473, 45 (201 x 67 and 333 x 111 below
     // level 1) 2060 -> 2072; 105 (450 x 151) 2760 -> 2702.
-    const int nu = std::max(B.nu_down, B.nu_up);
+    // A cell-weight level gains from the same tiles, on which a node's row is built once instead
+    // of once per sweep (640 x 320 cells: FP64 2962 -> 2849, mixed 2632 -> 2594; 1440 x 240 FP64
+    // 4122 -> 3911; 1600 x 560 4099 -> 3999 and 3296 -> 3173; 3000 x 1000 FP64 8838 -> 8617), up
+    // to 2000 of them, from where the halo counts (3948: mixed 6950 -> 7156), and in FP64, where
+    // two workgroups fit a CU, unless the second round of workgroups is half empty (646: 3174 ->
+    // 3224 with 1200 x 400 cells).
+    const int nu = std::max(B.nu_down, B.nu_up), n = band_tiles(L.nx, L.ny, 16, 12);
     if (band_ext(16, nu, true) * band_ext(12, nu, true) <= (size_t)kBandThreadsMid &&
         band_lds_bytes(16, 12, nu, h.bs_, sizeof(T), B.src, true) <= kBandLdsBytes &&
-        band_tiles(L.nx, L.ny, 16, 12) >= kBandMidTiles) {
+        n >= kBandMidTiles &&
+        (B.src == kSrcStencil || (n <= 2000 && !(sizeof(T) == 8 && n > 512 && n <= 768)))) {
       B.tx = 16;
       B.ty = 12;
       B.wide = 2;
