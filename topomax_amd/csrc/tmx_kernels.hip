@@ -2785,16 +2785,20 @@ template hipError_t tail_vcycle<double, 2>(const TailDesc<double>&, hipStream_t)
 template hipError_t tail_vcycle<float, 1>(const TailDesc<float>&, hipStream_t);
 template hipError_t tail_vcycle<float, 2>(const TailDesc<float>&, hipStream_t);
 
-// Galerkin product R A P for tensor-product linear (bilinear) coarsening, one thread per
-// coarse node (I, J) and coarse stencil direction kc (nine threads per node): the thread forms
-// the coarse block A_c(I,J)[kc] = sum over fine rows f near (I, J) and their stencil neighbours
-// g of P(f,I) A_f(f,g) P(g, (I,J)+kc).  The fine nodes f that interpolate from (I, J) lie
-// within one node of its fine position p, and their stencil neighbours g within two; the 1-D
-// interpolation weights from those five fine positions per axis to the three coarse positions
-// I-1..I+1 (and J-1..J+1) are tabulated, so every loop has compile-time trip counts and
-// indices: the 9 x 9 stencil entries of the 3 x 3 fine rows are loaded unconditionally (rows
-// clamped into the grid; their weight is zero then).  The nine threads of a node read the
-// same fine entries (cache hits), and the per-thread work is a ninth of a node's.
+// Galerkin product R A P for tensor-product linear (bilinear) coarsening, one thread per coarse
+// node (I, J) and entry e of the BS x BS blocks (one e per workgroup): the thread forms the
+// entries A_c(I,J)[kc] of all nine coarse directions kc as the sum over fine rows f near (I, J)
+// and their stencil neighbours g of P(f,I) A_f(f,g) P(g, (I,J)+kc).  The fine nodes f that
+// interpolate from (I, J) lie within one node of its fine position p, and their stencil
+// neighbours g within two; the 1-D interpolation weights from those five fine positions per axis
+// to the three coarse positions I-1..I+1 (and J-1..J+1) are tabulated, so every loop has
+// compile-time trip counts and indices, and the combinations that no grid uses drop out (169 of
+// 729 products stay).  The rows are loaded unconditionally (clamped into the grid; their weight
+// is zero then), 27 values at a time.
+// Bound by these loads: 81 a thread, each a wave's run of every second fine node.  One thread
+// per (node, kc) instead, reading all blocks' entries, made a wave's load fetch 7 nodes, and the
+// nine threads of a node each loaded them all.  499 x 167 cells from 999 x 333 139 -> 34.6 us,
+// 250 x 84 from those 42.6 -> 11.6, small levels 12.5-13.4 -> 5.0-5.8; the sums keep their order.
 template <int BS>
 __device__ __forceinline__ void stencil_rap_body(const BlkId blk, int nxf,
                                                  int nyf,
@@ -2805,66 +2809,72 @@ __device__ __forceinline__ void stencil_rap_body(const BlkId blk, int nxf,
                                                  double* stc, float* stc32) {
   const unsigned nnf = (unsigned)(nxf + 1) * (unsigned)(nyf + 1);
   const unsigned nnc = (unsigned)(nxc + 1) * (unsigned)(nyc + 1);
-  const unsigned t = blk.id * blockDim.x + threadIdx.x;
-  const unsigned i = t / 9u;
-  const int kc = (int)(t - 9u * i);
+  constexpr int B2 = BS * BS;
+  const int e = (int)(blk.id % (unsigned)B2);  // entry of the blocks, one per workgroup
+  const unsigned i = blk.id / (unsigned)B2 * 64u + threadIdx.x;
   if (i >= nnc) return;
   const int I = (int)(i % (unsigned)(nxc + 1)), J = (int)(i / (unsigned)(nxc + 1));
-  constexpr int B2 = BS * BS;
-  double acc[B2];
+  double acc[9];
 #pragma unroll
-  for (int e = 0; e < B2; ++e) acc[e] = 0.0;
+  for (int kc = 0; kc < 9; ++kc) acc[kc] = 0.0;
   const int px = cpos(I, nxf, nxc), py = cpos(J, nyf, nyc);
-  const int dxc = kc % 3, dyc = kc / 3;  // coarse neighbour (I-1+dxc, J-1+dyc)
-  // wx[a]: weight of coarse column I-1+dxc at fine column px-2+a (zero outside the grid);
-  // wx1[a]: weight of coarse column I at it (the row side of R)
-  float wx[5], wy[5], wx1[5], wy1[5];
+  // wx[d][a]: weight of coarse column I-1+d at fine column px-2+a (zero outside the grid);
+  // only d = 0: a = 0, 1; d = 1: a = 1, 2, 3; d = 2: a = 3, 4 can be nonzero where the row side
+  // of R is too
+  double wx[3][5], wy[3][5];
 #pragma unroll
   for (int a = 0; a < 5; ++a) {
     const int gx = px - 2 + a, gy = py - 2 + a;
     const bool ox = gx < 0 || gx > nxf, oy = gy < 0 || gy > nyf;
-    // one interpolation stencil per fine position, read for both coarse columns (rows)
     const Interp1 rx = interp1(gx, nxf, nxc), ry = interp1(gy, nyf, nyc);
     auto wof = [](const Interp1& r, int c) {
-      return (float)((r.c[0] == c ? r.w[0] : 0.0) + (r.n > 1 && r.c[1] == c ? r.w[1] : 0.0));
+      return (r.c[0] == c ? r.w[0] : 0.0) + (r.n > 1 && r.c[1] == c ? r.w[1] : 0.0);
     };
-    wx[a] = ox ? 0.f : wof(rx, I - 1 + dxc);
-    wy[a] = oy ? 0.f : wof(ry, J - 1 + dyc);
-    wx1[a] = ox ? 0.f : wof(rx, I);
-    wy1[a] = oy ? 0.f : wof(ry, J);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      wx[d][a] = ox ? 0.0 : wof(rx, I - 1 + d);
+      wy[d][a] = oy ? 0.0 : wof(ry, J - 1 + d);
+    }
   }
   const bool self_fixed = node_fixed(fixed, I, J, nxc, nyc);
-  const bool live = !node_fixed(fixed, I - 1 + dxc, J - 1 + dyc, nxc, nyc);
-  if (!self_fixed && live) {
+  if (!self_fixed) {
+    const double* st = stf + (size_t)e * nnf;
 #pragma unroll
-    for (int fyi = 0; fyi < 3; ++fyi)
+    for (int fyi = 0; fyi < 3; ++fyi) {
+      // the rows of three fine nodes (px-1+fxi, py-1+fyi), all their loads in flight at once
+      const int fy = min(max(py - 1 + fyi, 0), nyf);
+      double v[3][9];
 #pragma unroll
       for (int fxi = 0; fxi < 3; ++fxi) {
-        // fine row f = (px-1+fxi, py-1+fyi): table index fxi+1, fyi+1
-        const double wf = (double)(wx1[fxi + 1] * wy1[fyi + 1]);
-        const int fx = min(max(px - 1 + fxi, 0), nxf), fy = min(max(py - 1 + fyi, 0), nyf);
+        const int fx = min(max(px - 1 + fxi, 0), nxf);
         const unsigned f = (unsigned)fy * (unsigned)(nxf + 1) + (unsigned)fx;
-        // the fine row's 9 B2 entries, all loads in flight before the first is used
-        double v[9 * B2];
 #pragma unroll
-        for (int q = 0; q < 9 * B2; ++q) v[q] = stf[(size_t)q * nnf + f];
+        for (int k = 0; k < 9; ++k) v[fxi][k] = st[(size_t)(k * B2) * nnf + f];
+      }
+#pragma unroll
+      for (int fxi = 0; fxi < 3; ++fxi) {
+        const double wf = wx[1][fxi + 1] * wy[1][fyi + 1];
 #pragma unroll
         for (int k = 0; k < 9; ++k) {
           const int ax = fxi + k % 3, ay = fyi + k / 3;  // neighbour g at table index (ax, ay)
-          const double w = wf * (double)(wx[ax] * wy[ay]);
 #pragma unroll
-          for (int e = 0; e < B2; ++e) acc[e] += w * v[k * B2 + e];
+          for (int kc = 0; kc < 9; ++kc) {
+            const int dx = kc % 3, dy = kc / 3;  // coarse neighbour (I-1+dx, J-1+dy)
+            if (ax < 2 * dx - (dx > 0) || ax > 2 * dx + 1) continue;
+            if (ay < 2 * dy - (dy > 0) || ay > 2 * dy + 1) continue;
+            acc[kc] += wf * (wx[dx][ax] * wy[dy][ay]) * v[fxi][k];
+          }
         }
       }
+    }
   }
-  if (self_fixed && kc == 4) {
+  if (self_fixed && e % (BS + 1) == 0) acc[4] = 1.0;
 #pragma unroll
-    for (int a = 0; a < BS; ++a) acc[a * BS + a] = 1.0;
-  }
-#pragma unroll
-  for (int e = 0; e < B2; ++e) {
-    stc[(size_t)(kc * B2 + e) * nnc + i] = acc[e];
-    if (stc32) stc32[(size_t)(kc * B2 + e) * nnc + i] = (float)acc[e];
+  for (int kc = 0; kc < 9; ++kc) {
+    const bool live = kc == 4 || !node_fixed(fixed, I - 1 + kc % 3, J - 1 + kc / 3, nxc, nyc);
+    const double o = live ? acc[kc] : 0.0;
+    stc[(size_t)(kc * B2 + e) * nnc + i] = o;
+    if (stc32) stc32[(size_t)(kc * B2 + e) * nnc + i] = (float)o;
   }
 }
 
@@ -2880,7 +2890,8 @@ hipError_t stencil_rap(int nxf, int nyf, int nxc, int nyc, int nested, unsigned 
                        const double* stf, double* stc, hipStream_t s, float* stc32) {
   if (nested) return hipErrorInvalidValue;  // 9-point levels are always bilinear coarsenings
   if ((size_t)(nxf + 1) * (nyf + 1) >= (1ull << 31)) return hipErrorInvalidValue;
-  TMX_LAUNCH_OR_RECORD(64, (stencil_rap_body<BS>), grid1d(9 * (size_t)(nxc + 1) * (nyc + 1), 64), 0, s, (k_stencil_rap<BS>), nxf, nyf, nxc, nyc, fixed, stf, stc, stc32);
+  TMX_LAUNCH_OR_RECORD(64, (stencil_rap_body<BS>), BS * BS * grid1d((size_t)(nxc + 1) * (nyc + 1), 64), 0, s,
+                       (k_stencil_rap<BS>), nxf, nyf, nxc, nyc, fixed, stf, stc, stc32);
   return hipGetLastError();
 }
 template hipError_t stencil_rap<1>(int, int, int, int, int, unsigned, const double*, double*,
