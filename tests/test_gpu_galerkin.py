@@ -13,10 +13,13 @@ from tests.cases import CANTILEVER, gpu_problem
 pytestmark = pytest.mark.gpu
 
 # one product to the coarsest grid (at most 64 nodes), then two and three
-GRIDS = [(9, 7), (13, 9), (14, 9), (9, 14), (1, 40), (41, 1), (2, 33), (3, 31), (45, 15), (63, 23)]
+GRIDS = [(9, 7), (13, 9), (14, 9), (9, 14), (1, 40), (41, 1), (2, 33), (3, 31), (45, 15), (63, 23), (29, 21), (41, 33), (33, 65)]
 
 
-def interpolation(n, nc):
+def interpolation(n, nc, finest):
+    """Cells are paired from the near and the far side on alternate levels."""
+    if n > 1 and n % 2 and ((n - 1).bit_length() - (finest - 1).bit_length()) % 2:
+        return interpolation(n, nc, n)[::-1, ::-1]
     p = np.zeros((n + 1, nc + 1))
     for f in range(n + 1):
         if n == nc:
@@ -61,7 +64,7 @@ def test_galerkin_products(nx, ny, fixed):
     cx, cy = nx, ny
     while (cx + 1) * (cy + 1) > 64:
         mx, my = (cx + 1) // 2, (cy + 1) // 2
-        I = np.kron(np.kron(interpolation(cy, my), interpolation(cx, mx)), np.eye(2))
+        I = np.kron(np.kron(interpolation(cy, my, ny), interpolation(cx, mx, nx)), np.eye(2))
         P = (P @ I) * free(mx, my)
         cx, cy = mx, my
     keep = free(cx, cy) > 0

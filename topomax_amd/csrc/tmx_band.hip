@@ -339,8 +339,11 @@ __device__ __forceinline__ void band_pass(const BandLevel<T>& L, BandNode<T, BS,
 
 // coarse nodes whose restriction centre lies in fine nodes [X0, X1) of one direction
 __device__ __forceinline__ void band_coarse_range(int X0, int X1, int nf, int nc, int& lo,
-                                                  int& hi) {
-  if (nf == nc) {
+                                                  int& hi, bool m) {
+  if (m) {  // (centres 0, 1, 3, 5, ..., nf)
+    lo = X0 > 0 ? (X0 + 2) >> 1 : 0;
+    hi = min((X1 + 2) >> 1, nc + 1);
+  } else if (nf == nc) {
     lo = X0;
     hi = min(X1, nf + 1);
   } else {
@@ -452,8 +455,9 @@ __device__ __forceinline__ void band_down_body(const BlkId blk, const BandLevel<
   __syncthreads();
   // restriction of the residual to the owned coarse nodes
   int I0, I1, J0, J1;
-  band_coarse_range(X0, X0 + L.tx, L.nx, L.nxc, I0, I1);
-  band_coarse_range(Y0, Y0 + L.ty, L.ny, L.nyc, J0, J1);
+  const bool mx = mirrored(L.fixed, 0, L.nx), my = mirrored(L.fixed, 1, L.ny);
+  band_coarse_range(X0, X0 + L.tx, L.nx, L.nxc, I0, I1, mx);
+  band_coarse_range(Y0, Y0 + L.ty, L.ny, L.nyc, J0, J1, my);
   const T* r = nxt;
   if (I1 > I0) for_region<NT>(I1 - I0, J1 - J0, [&](int rx, int ry) {
     const int I = I0 + rx, J = J0 + ry;
@@ -472,15 +476,15 @@ __device__ __forceinline__ void band_down_body(const BlkId blk, const BandLevel<
           acc[q] = r[BS * i + q] + T(0.5) * sum;
         }
       } else {
-        const int px = cpos(I, L.nx, L.nxc), py = cpos(J, L.ny, L.nyc);
+        const int px = cpos(I, L.nx, L.nxc, mx), py = cpos(J, L.ny, L.nyc, my);
 #pragma unroll
         for (int dy = -1; dy <= 1; ++dy) {
           const int fy = py + dy;
-          const double wy = (fy < 0 || fy > L.ny) ? 0.0 : interp1_weight(fy, L.ny, L.nyc, J);
+          const double wy = (fy < 0 || fy > L.ny) ? 0.0 : interp1_weight(fy, L.ny, L.nyc, J, my);
 #pragma unroll
           for (int dx = -1; dx <= 1; ++dx) {
             const int fx = px + dx;
-            const double w = (fx < 0 || fx > L.nx) ? 0.0 : wy * interp1_weight(fx, L.nx, L.nxc, I);
+            const double w = (fx < 0 || fx > L.nx) ? 0.0 : wy * interp1_weight(fx, L.nx, L.nxc, I, mx);
             const int i = (fy - OY) * EX + (fx - OX);
 #pragma unroll
             for (int q = 0; q < BS; ++q) acc[q] += (T)w * r[BS * i + q];
@@ -543,7 +547,8 @@ __device__ __forceinline__ void band_up_body(const BlkId blk, const BandLevel<T>
               for (int q = 0; q < BS; ++q)
                 xv[u][q] += T(0.5) * (ec[BS * c0 + q] + ec[BS * c1 + q]);
             } else {
-              const Interp1 ix = interp1(gx, L.nx, L.nxc), iy = interp1(gy, L.ny, L.nyc);
+              const Interp1 ix = interp1(gx, L.nx, L.nxc, mirrored(L.fixed, 0, L.nx));
+              const Interp1 iy = interp1(gy, L.ny, L.nyc, mirrored(L.fixed, 1, L.ny));
               const unsigned cx1 = ix.n > 1 ? ix.c[1] : ix.c[0];
               const unsigned cy1 = iy.n > 1 ? iy.c[1] : iy.c[0];
               const T wx0 = (T)ix.w[0], wx1 = ix.n > 1 ? (T)ix.w[1] : T(0);

@@ -213,8 +213,22 @@ struct Interp1 {
   double w[2];
 };
 
-__device__ __forceinline__ Interp1 interp1(int f, int nf, int nc) {
+// Whether a level of nf cells along axis (0: x, 1: y) pairs them from the far side, so that an odd
+// count leaves its single cell at the near side.  With pairs from the near side on every level
+// a far column of cells stays one fine cell wide while all others double, and the smoother
+// fails on the anisotropy (mixed, rtol 1e-10, PCG iterations: 771 x 257 cells 31, 483 x 161 31,
+// 1350 x 450 30, against 15 or 16 with even levels).  The bit length of nf - 1 falls by one from
+// each level to the next, whichever of them are odd, so its parity alternates the sides; the
+// finest level pairs from the near side.  The same meshes then take 19, 18 and 18, 999 x 333
+// 15 for 20, 1731 x 577 19 for 41; whole steps FP64 333 x 111 cells 2030 -> 1897 us, mixed
+// 999 x 333 3497 -> 2921.
+__device__ __forceinline__ bool mirrored(unsigned fixed, int axis, int nf) {
+  return (nf & 1) && nf > 1 && (((32u - __clz(nf - 1)) ^ (fixed >> kMirrorBit[axis])) & 1u);
+}
+
+__device__ __forceinline__ Interp1 interp1(int f, int nf, int nc, bool m) {
   Interp1 r;
+  if (m) f = nf - f;  // (the same from the far side)
   if (nf == nc) {  // not coarsened in this direction
     r.n = 1; r.c[0] = f; r.w[0] = 1.0;
   } else if ((f & 1) == 0) {
@@ -224,13 +238,20 @@ __device__ __forceinline__ Interp1 interp1(int f, int nf, int nc) {
   } else {
     r.n = 2; r.c[0] = (f - 1) >> 1; r.c[1] = (f + 1) >> 1; r.w[0] = r.w[1] = 0.5;
   }
+  if (m) {
+    r.c[0] = nc - r.c[0];
+    if (r.n > 1) r.c[1] = nc - r.c[1];
+  }
   return r;
 }
 
-__device__ __forceinline__ int cpos(int I, int nf, int nc) { return nf == nc ? I : min(2 * I, nf); }
+// fine position of coarse node I
+__device__ __forceinline__ int cpos(int I, int nf, int nc, bool m) {
+  return nf == nc ? I : m ? max(2 * I - 1, 0) : min(2 * I, nf);
+}
 
-__device__ __forceinline__ double interp1_weight(int f, int nf, int nc, int I) {
-  const Interp1 r = interp1(f, nf, nc);
+__device__ __forceinline__ double interp1_weight(int f, int nf, int nc, int I, bool m) {
+  const Interp1 r = interp1(f, nf, nc, m);
   return (r.c[0] == I ? r.w[0] : 0.0) + (r.n > 1 && r.c[1] == I ? r.w[1] : 0.0);
 }
 

@@ -13,6 +13,9 @@ namespace tmx {
 
 // Dirichlet side bits (same values as TMX_FIX_* in include/tmx.h)
 enum SideBits : unsigned { kLeft = 1u, kRight = 2u, kTop = 4u, kBottom = 8u };
+// beside them: the parity, per axis, of the levels that pair their cells from the far side (see
+// `mirrored`)
+constexpr int kMirrorBit[2] = {8, 9};
 
 // Deterministic two-stage reductions: a kernel writes one partial per block into
 // `partials` (kMaxPartials doubles) and records the block count; a one-block kernel adds them.

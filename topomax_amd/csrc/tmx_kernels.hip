@@ -2147,15 +2147,16 @@ __device__ __forceinline__ void restrict_bilinear_node(int nxf, int nyf, int nxc
   double acc[BS];
 #pragma unroll
   for (int q = 0; q < BS; ++q) acc[q] = 0.0;
-  const int px = cpos(I, nxf, nxc), py = cpos(J, nyf, nyc);
+  const bool mx = mirrored(fixed, 0, nxf), my = mirrored(fixed, 1, nyf);
+  const int px = cpos(I, nxf, nxc, mx), py = cpos(J, nyf, nyc, my);
 #pragma unroll
   for (int dy = -1; dy <= 1; ++dy) {
     const int fy = py + dy;
-    const double wy = (fy < 0 || fy > nyf) ? 0.0 : interp1_weight(fy, nyf, nyc, J);
+    const double wy = (fy < 0 || fy > nyf) ? 0.0 : interp1_weight(fy, nyf, nyc, J, my);
 #pragma unroll
     for (int dx = -1; dx <= 1; ++dx) {
       const int fx = px + dx;
-      const double w = (fx < 0 || fx > nxf) ? 0.0 : wy * interp1_weight(fx, nxf, nxc, I);
+      const double w = (fx < 0 || fx > nxf) ? 0.0 : wy * interp1_weight(fx, nxf, nxc, I, mx);
       const size_t g = (size_t)min(max(fy, 0), nyf) * (nxf + 1) + min(max(fx, 0), nxf);
 #pragma unroll
       for (int q = 0; q < BS; ++q) acc[q] += w * (double)rf[BS * g + q];
@@ -2172,7 +2173,8 @@ __device__ __forceinline__ void prolong_bilinear_node(int nxf, int nyf, int nxc,
                                                       T* __restrict__ xf, size_t i) {
   const int fx = (int)((unsigned)i % (unsigned)(nxf + 1)), fy = (int)((unsigned)i / (unsigned)(nxf + 1));
   if (node_fixed(fixed, fx, fy, nxf, nyf)) return;
-  const Interp1 ix = interp1(fx, nxf, nxc), iy = interp1(fy, nyf, nyc);
+  const Interp1 ix = interp1(fx, nxf, nxc, mirrored(fixed, 0, nxf));
+  const Interp1 iy = interp1(fy, nyf, nyc, mirrored(fixed, 1, nyf));
   const int cx0 = ix.c[0], cx1 = ix.n > 1 ? ix.c[1] : ix.c[0];
   const int cy0 = iy.c[0], cy1 = iy.n > 1 ? iy.c[1] : iy.c[0];
   const double wx0 = ix.w[0], wx1 = ix.n > 1 ? ix.w[1] : 0.0;
@@ -2200,15 +2202,16 @@ __device__ __forceinline__ void s9_resrestrict_node(int nxf, int nyf, int nxc, i
 #pragma unroll
   for (int q = 0; q < BS; ++q) acc[q] = 0.0;
   if (!node_fixed(fixed, I, J, nxc, nyc)) {
-    const int px = cpos(I, nxf, nxc), py = cpos(J, nyf, nyc);
+    const bool mx = mirrored(fixed, 0, nxf), my = mirrored(fixed, 1, nyf);
+  const int px = cpos(I, nxf, nxc, mx), py = cpos(J, nyf, nyc, my);
     for (int dy = -1; dy <= 1; ++dy) {
       const int fy = py + dy;
       if (fy < 0 || fy > nyf) continue;
-      const double wy = interp1_weight(fy, nyf, nyc, J);
+      const double wy = interp1_weight(fy, nyf, nyc, J, my);
       for (int dx = -1; dx <= 1; ++dx) {
         const int fx = px + dx;
         if (fx < 0 || fx > nxf) continue;
-        const double w = wy * interp1_weight(fx, nxf, nxc, I);
+        const double w = wy * interp1_weight(fx, nxf, nxc, I, mx);
         if (w == 0.0) continue;
         const size_t f = (size_t)fy * (nxf + 1) + fx;
         T r[BS];
@@ -2242,7 +2245,8 @@ __device__ __forceinline__ void corrected(int nxf, int nyf, int nxc, int nyc, un
 #pragma unroll
   for (int q = 0; q < BS; ++q) out[q] = x[BS * f + q];
   if (node_fixed(fixed, fx, fy, nxf, nyf)) return;
-  const Interp1 ix = interp1(fx, nxf, nxc), iy = interp1(fy, nyf, nyc);
+  const Interp1 ix = interp1(fx, nxf, nxc, mirrored(fixed, 0, nxf));
+  const Interp1 iy = interp1(fy, nyf, nyc, mirrored(fixed, 1, nyf));
   for (int bb = 0; bb < iy.n; ++bb)
     for (int aa = 0; aa < ix.n; ++aa) {
       const T w = (T)(ix.w[aa] * iy.w[bb]);
@@ -2462,17 +2466,28 @@ struct TailNode {
   }
 };
 
+// one axis of a level: m = 1 if mirrored, end: the node that lies on its coarse node alone (an odd
+// count's last, or first if mirrored), whose neighbour is not half way
+struct TailAxis {
+  int m, end;
+  __device__ __forceinline__ TailAxis(unsigned fixed, int axis, int nf)
+      : m(mirrored(fixed, axis, nf) ? 1 : 0), end(m ? 0 : nf) {}
+};
+
 // The bilinear transfers between two levels (coarse cells = ceil(fine / 2) per axis): an even
 // fine node lies on coarse node f / 2, the last node of an odd count on the last coarse node,
-// any other odd node half way.  Restriction at coarse node I: its fine node p = min(2I, nf) and
-// the halves from p - 1 and p + 1 that lie half way (the border is zero).  Products with 0, 1/2
+// any other odd node half way; mirrored (see `mirrored`) the same counted from the far side.
+// Restriction at coarse node I: its fine node p and the halves from p - 1 and p + 1 that lie half
+// way (the border is zero).  Products with 0, 1/2
 // and 1 are exact; the sum is kept in double, as in the launch-per-step transfers.
 template <typename T, int BS>
 __device__ __forceinline__ TailVal<T, BS> tail_restrict(const TailGeom& f, const TailVal<T, BS>* rf,
-                                                        int I, int J, bool fixed) {
-  const int px = min(2 * I, f.nx), py = min(2 * J, f.ny);
-  const double wx[3] = {(px & 1) ? 0.0 : 0.5, 1.0, ((px & 1) || px + 1 == f.nx) ? 0.0 : 0.5};
-  const double wy[3] = {(py & 1) ? 0.0 : 0.5, 1.0, ((py & 1) || py + 1 == f.ny) ? 0.0 : 0.5};
+                                                        int I, int J, bool fixed, TailAxis ax,
+                                                        TailAxis ay) {
+  const int px = min(max(2 * I - ax.m, 0), f.nx), py = min(max(2 * J - ay.m, 0), f.ny);
+  const double hx = ((px ^ ax.m) & 1) ? 0.0 : 0.5, hy = ((py ^ ay.m) & 1) ? 0.0 : 0.5;
+  const double wx[3] = {px - 1 == ax.end ? 0.0 : hx, 1.0, px + 1 == ax.end ? 0.0 : hx};
+  const double wy[3] = {py - 1 == ay.end ? 0.0 : hy, 1.0, py + 1 == ay.end ? 0.0 : hy};
   const TailVal<T, BS>* c = rf + (py + 1) * f.pitch + px + 1;
   double acc[BS];
 #pragma unroll
@@ -2495,14 +2510,14 @@ __device__ __forceinline__ TailVal<T, BS> tail_restrict(const TailGeom& f, const
 // xf += P ec at the fine node (ix, iy); ec: coarse node (0, 0), rows of cp nodes
 template <typename T, int BS>
 __device__ __forceinline__ void tail_prolong(const TailGeom& f, int ix, int iy,
-                                             const TailVal<T, BS>* ec, int cp,
-                                             TailVal<T, BS>& xf) {
-  const T x1 = (ix & 1) ? (ix == f.nx ? T(1) : T(0.5)) : T(0), x0 = T(1) - x1;
-  const T y1 = (iy & 1) ? (iy == f.ny ? T(1) : T(0.5)) : T(0), y0 = T(1) - y1;
-  // (an even node's second neighbour has weight zero and may not exist: its own is read)
-  const int ox = (ix & 1) ? 1 : 0, oy = (iy & 1) ? cp : 0;
-  const TailVal<T, BS>* e = ec + (iy >> 1) * cp + (ix >> 1);
-  const TailVal<T, BS> e00 = e[0], e10 = e[ox], e01 = e[oy], e11 = e[oy + ox];
+                                             const TailVal<T, BS>* ec, int cp, TailAxis ax,
+                                             TailAxis ay, TailVal<T, BS>& xf) {
+  // (a node with one neighbour alone reads another with weight zero, itself or one in range)
+  const int ox = (ix ^ ax.m) & 1, oy = (iy ^ ay.m) & 1;
+  const T x1 = ox ? (ix == ax.end ? T(1 - ax.m) : T(0.5)) : T(0), x0 = T(1) - x1;
+  const T y1 = oy ? (iy == ay.end ? T(1 - ay.m) : T(0.5)) : T(0), y0 = T(1) - y1;
+  const TailVal<T, BS>* e = ec + ((iy + ay.m) >> 1) * cp + ((ix + ax.m) >> 1);
+  const TailVal<T, BS> e00 = e[0], e10 = e[ox], e01 = e[oy * cp], e11 = e[oy * cp + ox];
   TailVal<T, BS> x = xf;
 #pragma unroll
   for (int q = 0; q < BS; ++q)
@@ -2631,10 +2646,12 @@ __device__ __forceinline__ void tail_vcycle_body(const BlkId blk, const TailDesc
     V* const b1 = reinterpret_cast<V*>(lds + off + padded);
     const V* b = reinterpret_cast<const V*>(lds + off + 2 * padded);
     int w = w_mid;
+    const TailAxis mx(fixed, 0, g.nx), my(fixed, 1, g.ny);
 #pragma unroll
     for (int k = 0; k < kPer; ++k)
       if (nodes[k].live && !node_fixed(fixed, nodes[k].ix, nodes[k].iy, g.nx, g.ny))
-        tail_prolong<T, BS>(g, nodes[k].ix, nodes[k].iy, ec, cp, (w ? b1 : b0)[nodes[k].at]);
+        tail_prolong<T, BS>(g, nodes[k].ix, nodes[k].iy, ec, cp, mx, my,
+                            (w ? b1 : b0)[nodes[k].at]);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kPer; ++k) nodes[k].finish();  // (rows requested before the call)
@@ -2651,6 +2668,7 @@ __device__ __forceinline__ void tail_vcycle_body(const BlkId blk, const TailDesc
   for (int l = 0; l + 1 < nl; ++l) {
     const TailGeom g(d.lev[l]), c(d.lev[l + 1]);
     const int off = d.lev[l].off, padded = d.lev[l].padded, coff = d.lev[l + 1].off;
+    const TailAxis mx(fixed, 0, g.nx), my(fixed, 1, g.ny);
     const bool rows = l + 2 < nl;  // (the dense coarsest has none)
     const T* cst = d.lev[l + 1].st;
     spare = l == 0 ? down(std::integral_constant<int, 2>(), top, rt, g, off, padded)
@@ -2663,13 +2681,13 @@ __device__ __forceinline__ void tail_vcycle_body(const BlkId blk, const TailDesc
       __syncthreads();
       if (low[0].live)
         rl[0] = tail_restrict<T, BS>(g, spare, low[0].ix, low[0].iy,
-                                     node_fixed(fixed, low[0].ix, low[0].iy, c.nx, c.ny));
+                                     node_fixed(fixed, low[0].ix, low[0].iy, c.nx, c.ny), mx, my);
     } else {
       __syncthreads();
       const int J = (int)(((unsigned)tid * c.div) >> 20), I = tid - J * (c.nx + 1);
       if (J <= c.ny)  // (at most 128 nodes)
         reinterpret_cast<V*>(lds + coff)[tid] =
-            tail_restrict<T, BS>(g, spare, I, J, node_fixed(fixed, I, J, c.nx, c.ny));
+            tail_restrict<T, BS>(g, spare, I, J, node_fixed(fixed, I, J, c.nx, c.ny), mx, my);
       __syncthreads();
     }
   }
@@ -2817,7 +2835,8 @@ __device__ __forceinline__ void stencil_rap_body(const BlkId blk, int nxf,
   double acc[9];
 #pragma unroll
   for (int kc = 0; kc < 9; ++kc) acc[kc] = 0.0;
-  const int px = cpos(I, nxf, nxc), py = cpos(J, nyf, nyc);
+  const bool mx = mirrored(fixed, 0, nxf), my = mirrored(fixed, 1, nyf);
+  const int px = cpos(I, nxf, nxc, mx), py = cpos(J, nyf, nyc, my);
   // wx[d][a]: weight of coarse column I-1+d at fine column px-2+a (zero outside the grid);
   // only d = 0: a = 0, 1; d = 1: a = 1, 2, 3; d = 2: a = 3, 4 can be nonzero where the row side
   // of R is too
@@ -2826,7 +2845,7 @@ __device__ __forceinline__ void stencil_rap_body(const BlkId blk, int nxf,
   for (int a = 0; a < 5; ++a) {
     const int gx = px - 2 + a, gy = py - 2 + a;
     const bool ox = gx < 0 || gx > nxf, oy = gy < 0 || gy > nyf;
-    const Interp1 rx = interp1(gx, nxf, nxc), ry = interp1(gy, nyf, nyc);
+    const Interp1 rx = interp1(gx, nxf, nxc, mx), ry = interp1(gy, nyf, nyc, my);
     auto wof = [](const Interp1& r, int c) {
       return (r.c[0] == c ? r.w[0] : 0.0) + (r.n > 1 && r.c[1] == c ? r.w[1] : 0.0);
     };

@@ -82,7 +82,9 @@ int Hierarchy::init(Phys phys, int nx, int ny, double hx, double hy, unsigned fi
                     double mu, double eps, int coarse_max_nodes, hipStream_t s) {
   phys_ = phys;
   bs_ = phys == kElasticity ? 2 : 1;
-  fixed_ = fixed;
+  // (the finest level pairs its cells from the near side, see `mirrored`)
+  auto parity = [](int n) { int w = 0; for (n -= 1; n > 0; n >>= 1) ++w; return (unsigned)(w & 1); };
+  fixed_ = fixed | parity(nx) << kMirrorBit[0] | parity(ny) << kMirrorBit[1];
   lam_ = lam;
   mu_ = mu;
   eps_ = eps;
@@ -824,7 +826,8 @@ int Hierarchy::vcycle(int l, const T* b, T* out, hipStream_t s, RedSlot* dot_bz)
   const int rows_post = l == 0 ? pair_rows_post_[pi] : pair_rows_coarse_[1];
   const int rows_rr = l == 0 ? pair_rr_rows_[pi] : pair_rows_coarse_[2];
   const bool pair_pre = pair_level && rows_pre > 0 && npre >= 2;
-  const bool pair_fused = fused_ && pair_level;  // (nested or bilinear transfers)
+  // (nested transfers, or bilinear ones that pair from the near side)
+  const bool pair_fused = fused_ && pair_level && (l == 0 || C.nested_from_prev);
   const bool pair_post = pair_fused && rows_post > 0 && npost >= 2;
   const bool pair_rr = pair_pre && npre == 2 && pair_fused && rows_rr > 0;
   const int launches = npre - (pair_pre ? 1 : 0) + npost - (pair_post ? 1 : 0);
