@@ -95,7 +95,8 @@ typedef struct tmx_problem_desc {
 
 typedef struct tmx_solve_opts {
   double rtol;                /* relative residual |b - A u| / |b| */
-  int max_iter;               /* PCG iterations (inner, summed over refinements) */
+  int max_iter;               /* iterations (inner, summed over refinements), those of
+                                 MINRES included */
   int precision;              /* -1: handle default, else tmx_precision */
   double inner_rtol;          /* mixed: reduction asked of each FP32 inner solve */
   int max_outer;              /* mixed: refinement steps */
@@ -103,7 +104,8 @@ typedef struct tmx_solve_opts {
 
 typedef struct tmx_solve_stats {
   int iterations;             /* PCG iterations (all inner solves) */
-  int outer_iterations;       /* refinement steps (mixed), 1 for FP64 */
+  int outer_iterations;       /* refinement steps (mixed), 1 for FP64; one more when MINRES
+                                 took over from PCG */
   double rel_residual;        /* final |b - A u| / |b| */
   double setup_ms, solve_ms;  /* operator rebuild (device time on the solve's stream; with
                                  TMX_OPT_SETUP_OVERLAP the coarse part runs beside the solve

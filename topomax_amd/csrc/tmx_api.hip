@@ -423,7 +423,9 @@ static int p2_solve(tmx_problem* h, const double* xi, double* u, const SolvePara
   };
   // PCG on K2 d = r from r = F2, repeated on the true residual until |F2 - K2 u| <= rtol |F2|:
   // each run asks for half of what is missing, and two runs that gain less than 2x have met the
-  // residual's round-off floor.  What PCG does not solve goes to MINRES, from zero.
+  // residual's round-off floor.  What PCG does not solve goes to MINRES, from zero, with the
+  // iterations that are left of max_iter.
+  bool have_u = false;  // u holds a PCG iterate of true residual rel
   if (p2_apply_lanczos_ok(g)) {
     double* const r = P[0].get();
     double* const q = P[2].get();
@@ -492,10 +494,16 @@ static int p2_solve(tmx_problem* h, const double* xi, double* u, const SolvePara
         return done(TMX_ERR_NONFINITE);
       }
       if (rel <= prm.rtol) return done(TMX_OK);
+      have_u = true;
+      if (it >= prm.max_iter) {
+        set_error("PCG did not reach the tolerance within the iteration limit");
+        return done(TMX_ERR_NOT_CONVERGED);
+      }
       stalled = rel > 0.5 * best ? stalled + 1 : 0;
       best = std::min(best, rel);
-      if (stalled >= 2 || round >= 8 || it >= prm.max_iter) break;
+      if (stalled >= 2 || round >= 8) break;
     }
+    st->outer = 2;
   }
   // the operator launch also forms MINRES's first Lanczos update and the v.y partials
   MinresApplyL1 apply_l1 = nullptr;
@@ -507,11 +515,16 @@ static int p2_solve(tmx_problem* h, const double* xi, double* u, const SolvePara
       return 0;
     };
   int mr_its = 0;
+  double mr_rel = 0.0;
   const int rc = minres_core(h->ws, n, h->F2m.get(), X, bf, apply_fn, pc_fn, prm.rtol,
-                             prm.max_iter, bb, &mr_its, &rel, s,
+                             prm.max_iter - it, bb, &mr_its, &mr_rel, s,
                              std::getenv("TMX_TRACE") != nullptr, apply_l1);
   it += mr_its;
-  if (rc == TMX_OK || rc == TMX_ERR_NOT_CONVERGED) TMX_HIP(copy_vec<double>(n, X, u, s));
+  if (rc != TMX_OK && rc != TMX_ERR_NOT_CONVERGED) return done(rc);
+  if (!have_u || mr_rel < rel) {  // (the better of the two where neither reached the tolerance)
+    TMX_HIP(copy_vec<double>(n, X, u, s));
+    rel = mr_rel;
+  }
   return done(rc);
 }
 
