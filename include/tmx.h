@@ -261,7 +261,7 @@ enum tmx_option {
   TMX_OPT_BENCH_COLD = 26,      /* 1: tmx_bench_kernel times each launch alone after reading
                                    512 MiB (no inputs left in the caches); 0: back to back */
   TMX_OPT_RU_EVERY = 27,        /* TMX_MIXED_RU: iterations between residual replacements
-                                   (default 4; none once the residual nears the tolerance) */
+                                   (default 3; none once the residual nears the tolerance) */
   TMX_OPT_SETUP_OVERLAP = 28    /* 1 (default): an elasticity solve builds the coarse operators
                                    (Galerkin levels, coarsest inverse) on an internal stream
                                    while its first V-cycle smooths the finer levels; 0: in

@@ -265,7 +265,13 @@ class Hierarchy {
   // unlike a refinement restart.
   int pcg_ru(Workspace& ws, const double* b, double rtol, int max_iter, double* bnorm2,
              int* iters, double* rel, hipStream_t s);
-  int ru_every_ = 4;  // iterations between replacements
+  // Iterations between replacements.  Until it is replaced the FP32 residual's error stays at
+  // the size that it had when the residual was larger, so the period is bound by what an
+  // iteration gains, and one at which the recursion falls below that error pays with iterations.
+  // Iterations of a solve to 1e-8, period 2 / 3 / 4, beside the mixed scheme's: 1800 x 600 cells
+  // 14 / 15 / 16 (14), 2400 x 800 13 / 13 / 17 (13), 3000 x 1000 13 / 13 / 17 (13; steps 5289 /
+  // 5126 / 6097 us, mixed 5374); 333 x 111 10 / 10 / 11 (10), and 17 to 34 with period 5.
+  int ru_every_ = 3;
   // preconditioned MINRES (FP64, FP64 V-cycle) on A x = b from x0 = 0, restarted on the true
   // residual until |b - A x| <= rtol |b|; result in x_buf<double>().  For operators that are
   // not positive definite (PCG breakdown).
