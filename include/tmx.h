@@ -240,11 +240,16 @@ enum tmx_option {
                                    re-picks it per direction and precision); 0: the band
                                    kernels */
   TMX_OPT_FILTER_DCT = 21,      /* 2 (default): the filter's preconditioner (FP32 and FP64) is
-                                   the exact DCT-I / tridiagonal solver of
-                                   eps^2 K + (lumped mass) where 2 ny has no prime factor above
-                                   350 (FP64) or 450 (FP32), ny <= 2048 and nx + 1 <= 3072
-                                   (3-5 PCG iterations); 1: only where 2 ny has no prime factor
-                                   above 7; 0: the multigrid V-cycle */
+                                   an exact DCT-I / tridiagonal solver (3-5 PCG iterations) of
+                                   eps^2 K + the consistent mass averaged over the two ways to
+                                   draw the cells' diagonals, where ny <= 2048, nx + 1 <= 3072
+                                   and 2 ny has no prime factor above 7, or none above 350
+                                   (FP64) or 450 (FP32) with more than 1024 nodes; of the
+                                   latter, solves take it where it is estimated to be faster
+                                   than the V-cycle (few products of such primes per column,
+                                   eps well above the cell size); 1: of eps^2 K + the lumped
+                                   mass, where 2 ny has no prime factor above 7; 0: the
+                                   multigrid V-cycle */
   TMX_OPT_PAIR_LEVELS = 22,     /* elasticity element levels 0 .. value-1 run the paired
                                    column-strip kernels, the levels below them the band kernels
                                    (default 1: the finest only); 1..8 */
@@ -269,7 +274,8 @@ enum tmx_option {
 };
 int tmx_set_option(tmx_problem* h, int option, double value);
 /* One multigrid V-cycle z = M^-1 r (the PCG preconditioner).  which: 0 = elasticity with the
- * operator of xi (device, n_v), 1 = Helmholtz filter (xi ignored).  precision TMX_FP64 or
+ * operator of xi (device, n_v), 1 = Helmholtz filter (xi ignored), whose V-cycle is replaced by
+ * the DCT solver wherever TMX_OPT_FILTER_DCT allows it.  precision TMX_FP64 or
  * TMX_FP32 (r, z stay double). */
 int tmx_precondition(tmx_problem* h, int which, int precision, const double* xi,
                      const double* r, double* z);

@@ -55,18 +55,32 @@ class DctPrecond {
  public:
   // nx, ny: cells; 2 ny has no prime factor above max_prime (7 or kMaxPrime; above 7 on grids
   // of more than kMinNodesDirect nodes only), nx + 1 <= kMaxRow, and the FFT of 2 ny points fits
-  // the LDS budget; eps: the filter's length scale
+  // the LDS budget
   static bool supported(int nx, int ny, int max_prime);
+  // eps: the filter's length scale
   int init(int nx, int ny, double hx, double hy, double eps, hipStream_t s);
   // z = A'^-1 r (vectors of (nx + 1)(ny + 1) values; lumped: with the lumped mass in A'),
   // partials of r.z into rz if given
   int apply(const T* r, T* z, bool lumped, RedSlot* rz, hipStream_t s);
 
-  // Largest prime factor p of 2 ny: a prime without a butterfly costs p products per point
-  // (fft_stage_direct), the V-cycle the same per point whatever ny.  One filter solve to 1e-11,
-  // V-cycle / DCT in us: FP64 666 x 222 cells (p = 37) 978 / 304, 753 x 251 947 / 536, 933 x 311
-  // 974 / 791, 1203 x 401 1520 / 1646; FP32 954 / 275, 904 / 465, 907 / 662, 1377 / 1062 and
-  // 1503 x 503 1291 / 1392.
+  // Whether a filter solve with it is faster than with the V-cycle: always without direct stages;
+  // with them, by the estimated time of an iteration, in us, times the iterations.
+  //  - DCT: a direct stage of radix p takes p products a point (fft_stage_direct), in each
+  //    thread one after the other: 0.077 us for each of the p ceil(2 ny / 256) products, while a
+  //    CU has no more than one workgroup (two columns); several share the LDS.  The rest of an
+  //    iteration takes 43 + ny / 50.
+  //  - V-cycle: about 49 for 4000 nodes and 6 more for each doubling; 77 when the finest level
+  //    is coarsened to a nested one.
+  //  - iterations for eps/h = 1, 2, 5, 16, 50: DCT 7, 6, 5, 4, 3 (12 at 1/4), V-cycle 6 to 8.
+  // Solves of 9430 combinations of nx = 2 .. 2999, ny = 11 .. 2000 with a largest prime of 11 to
+  // 443, and eps/h = 1/4 .. 50 (seeded random rho, to 1e-11) take 0.6% more on average than with
+  // the faster of the two for each; 38% more with the V-cycle throughout, 25% with the DCT.
+  // V-cycle / DCT in us, FP64: 333 x 111 cells with eps/h = 8 (p = 37) 550 / 252, 512 x 257 with
+  // 16 702 / 542 and with 1.5 629 / 889, 16 x 257 with 16 426 / 558, 4 x 347 369 / 645,
+  // 512 x 1041 (p = 347) 1078 / 2000.
+  static bool pays(int nx, int ny, double hx, double hy, double eps);
+
+  // largest prime factor of 2 ny that has a direct stage
   static constexpr int kMaxPrime = sizeof(T) == 4 ? 450 : 350;
   // fewest nodes of a grid that such a prime's transform is used on: the V-cycle of a smaller
   // one is a few launches (33 x 11 cells 296 / 413, 66 x 22 490 / 352)

@@ -582,6 +582,30 @@ bool DctPrecond<T>::supported(int nx, int ny, int max_prime) {
 }
 
 template <typename T>
+bool DctPrecond<T>::pays(int nx, int ny, double hx, double hy, double eps) {
+  FftPlan p;
+  if (!fft_plan(2 * ny, kMaxPrime, p) || !p.direct) return true;
+  int per_point = 0;
+  for (int st = 0; st < p.nstages; ++st)
+    if (p.radix[st] > 7) per_point += p.radix[st];
+  const int work = per_point * ((2 * ny + kFftThreads<2> - 1) / kFftThreads<2>);
+  constexpr int kCus = 256;
+  const int per_cu = ((nx + 2) / 2 + kCus - 1) / kCus;  // workgroups of two columns
+  const double share = per_cu == 1 ? 1.0 : std::max(1.0, (sizeof(T) == 8 ? 0.8 : 0.5) * per_cu);
+  const double dct = 43.0 + ny / 50.0 + (sizeof(T) == 8 ? 5.0 : 3.0) * (per_cu - 1) +
+                     0.077 * work * share;
+  const double nodes = (double)(nx + 1) * (ny + 1);
+  const double vcycle = ((nx | ny) & 1 ? 49.0 : 77.0) +
+                        6.0 * std::max(-2.0, std::log2(nodes / 4000.0)) + 4e-5 * nodes;
+  // (a solve applies its preconditioner once more than it iterates)
+  const double l = std::log2(std::max(eps / std::sqrt(hx * hy), 0.2));
+  const double dct_its = l < 0.0 ? 8.0 - 2.5 * l
+                                 : std::max(sizeof(T) == 8 ? 4.0 : 4.5, 8.0 - 0.8 * l);
+  const double vcycle_its = std::min(9.0, 7.0 + 0.35 * std::max(0.0, l));
+  return 1.05 * dct * dct_its <= vcycle * vcycle_its;
+}
+
+template <typename T>
 int DctPrecond<T>::init(int nx, int ny, double hx, double hy, double eps, hipStream_t s) {
   if (!supported(nx, ny, kMaxPrime)) {
     set_error("internal: DCT preconditioner needs 2 ny with prime factors <= " +

@@ -224,9 +224,11 @@ class Hierarchy {
   template <typename T>
   int sweep_pair_rr0(int rows, const T* b, T* y, double om1, double om2, hipStream_t s,
                      int l = 0);
-  // z = M^-1 b; at level 0 the last smoothing sweep also writes partials of b.z to dot_bz
+  // z = M^-1 b; at level 0 the last smoothing sweep also writes partials of b.z to dot_bz.
+  // in_solve: the filter's DCT solver only where a solve is faster with it (DctPrecond::pays)
   template <typename T>
-  int vcycle(int l, const T* b, T* out, hipStream_t s, RedSlot* dot_bz = nullptr);
+  int vcycle(int l, const T* b, T* out, hipStream_t s, RedSlot* dot_bz = nullptr,
+             bool in_solve = false);
   // q = A p with p = z + beta p_old written to p_new; partials of p.q to dot.  z is read from
   // zlow (float) when that is given.
   // With xk, also xk += (*alpha) p_old (the previous iteration's deferred iterate update).
@@ -340,10 +342,12 @@ class Hierarchy {
   // filter_pipe_down / _up) with node-row chunks of these heights ([FP32, FP64][down, up]);
   // 0: band kernels
   int fpipe_rows_[2][2] = {{12, 12}, {12, 12}};
-  // filter preconditioner: the exact DCT-I / tridiagonal solver of the tensor-lumped
-  // operator (tmx_dct.h) instead of the V-cycle, where the grid allows it
-  // (0: never, 1: only where 2 ny has no prime factor above 7, 2: with larger primes too)
+  // filter preconditioner: the exact DCT-I / tridiagonal solver (tmx_dct.h) instead of the
+  // V-cycle, where the grid allows it (0: never; 1: of the operator with the lumped mass, only
+  // where 2 ny has no prime factor above 7; 2: with the averaged mass, with larger primes too,
+  // in solves where dct_pays_)
   int use_dct_ = 2;
+  bool dct_pays_[2] = {true, true};  // FP32, FP64 V-cycles
   std::unique_ptr<DctPrecond<float>> dct32_;
   std::unique_ptr<DctPrecond<double>> dct64_;
   template <typename T>

@@ -124,6 +124,10 @@ int Hierarchy::init(Phys phys, int nx, int ny, double hx, double hy, unsigned fi
     L.sh32 = SweepShape::make(L.nx, L.ny, rows_default(L.nx, L.ny));
   }
   find_tail();
+  if (phys_ == kFilter) {
+    dct_pays_[0] = DctPrecond<float>::pays(nx, ny, hx, hy, eps);
+    dct_pays_[1] = DctPrecond<double>::pays(nx, ny, hx, hy, eps);
+  }
   if (phys_ == kElasticity) {
     // Whole steps at rtol 1e-10 in us, chunks of 2 / 4 / 6 / 8 / 12 rows: FP64 600 x 200 cells
     // 2839 / 2830 / 2892 / 2941 / 3066, 1200 x 400 3911 / 3749 / 3622 / 3687 / 3642, 1800 x 600
@@ -758,7 +762,7 @@ static bool band_level(const Hierarchy& h, int l, BandLevel<T>& B) {
 }
 
 template <typename T>
-int Hierarchy::vcycle(int l, const T* b, T* out, hipStream_t s, RedSlot* dot_bz) {
+int Hierarchy::vcycle(int l, const T* b, T* out, hipStream_t s, RedSlot* dot_bz, bool in_solve) {
   const int last = (int)levels_.size() - 1;
   if (coarse_pending_ && l >= coarse_first_) TMX_TRY(join_coarse(s));
   if (l == last) {
@@ -768,6 +772,7 @@ int Hierarchy::vcycle(int l, const T* b, T* out, hipStream_t s, RedSlot* dot_bz)
   }
   if (use_tail_ && l == tail_ && l > 0) return tail_launch<T>(*this, b, out, s);
   if (l == 0 && phys_ == kFilter && use_dct_ && !use_graphs_ &&
+      (!in_solve || dct_pays_[sizeof(T) == 8]) &&
       DctPrecond<T>::supported(levels_[0].nx, levels_[0].ny,
                                use_dct_ == 1 ? 7 : DctPrecond<T>::kMaxPrime)) {
     auto& dct = dct_slot<T>();
@@ -977,13 +982,13 @@ T* Hierarchy::x_buf() {
 template <typename T, typename PC>
 static int enqueue_precondition(Hierarchy& h, RedSlot* rz, bool convert_r, hipStream_t s) {
   if constexpr (std::is_same<T, PC>::value) {
-    TMX_TRY(h.vcycle<T>(0, KrylovBufs<T>::r(h), KrylovBufs<T>::z(h), s, rz));
+    TMX_TRY(h.vcycle<T>(0, KrylovBufs<T>::r(h), KrylovBufs<T>::z(h), s, rz, true));
   } else {
     static_assert(std::is_same<T, double>::value && std::is_same<PC, float>::value,
                   "mixed PCG is FP64 Krylov with an FP32 V-cycle");
     const size_t nv = h.n();
     if (convert_r) TMX_HIP((convert<double, float>(nv, h.r64_.get(), h.r32_.get(), s)));
-    TMX_TRY(h.vcycle<float>(0, h.r32_.get(), h.z32_.get(), s, rz));
+    TMX_TRY(h.vcycle<float>(0, h.r32_.get(), h.z32_.get(), s, rz, true));
   }
   return 0;
 }
@@ -1767,7 +1772,7 @@ template int Hierarchy::sweep_pair_rr0<double>(int, const double*, double*, doub
                                                hipStream_t, int);
 template int Hierarchy::sweep_pair_rr0<float>(int, const float*, float*, double, double,
                                               hipStream_t, int);
-template int Hierarchy::vcycle<double>(int, const double*, double*, hipStream_t, RedSlot*);
-template int Hierarchy::vcycle<float>(int, const float*, float*, hipStream_t, RedSlot*);
+template int Hierarchy::vcycle<double>(int, const double*, double*, hipStream_t, RedSlot*, bool);
+template int Hierarchy::vcycle<float>(int, const float*, float*, hipStream_t, RedSlot*, bool);
 
 }  // namespace tmx
