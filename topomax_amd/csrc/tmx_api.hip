@@ -1053,7 +1053,7 @@ extern "C" int tmx_bench_kernel(tmx_problem* h, int kernel, int precision, int r
                                     e.x64_.get(), h->ws.sc() + kPcg.alpha);
     }
     if (kernel == 6) {  // zero-start pair with residual + restriction
-      if (!h->el.pair_post_ok()) return invalid("kernel 6 needs even nx and ny");
+      if (!h->el.pair_post_ok()) return invalid("kernel 6 needs a coarser level");
       const int rows = h->el.pair_rr_rows_[f64 ? 1 : 0];
       if (f64)
         return h->el.sweep_pair_rr0<double>(rows, h->Fm.get(), h->tmp64.get(), 0.5, 0.5, s);
@@ -1061,7 +1061,7 @@ extern "C" int tmx_bench_kernel(tmx_problem* h, int kernel, int precision, int r
     }
     if (kernel >= 3) {  // paired sweeps with the handle's chunk heights
       const int op1 = kernel == 3 ? kSmoothZero : kProlongSmooth;
-      if (kernel != 3 && !h->el.pair_post_ok()) return invalid("kernel 4 needs even nx and ny");
+      if (kernel != 3 && !h->el.pair_post_ok()) return invalid("kernel 4 needs a coarser level");
       const int rows = (kernel == 3 ? h->el.pair_rows_ : h->el.pair_rows_post_)[f64 ? 1 : 0];
       if (f64)
         return h->el.sweep_pair0<double>(op1, rows, h->u_s.get(), h->Fm.get(), h->tmp64.get(),
@@ -1122,7 +1122,7 @@ extern "C" int tmx_bench_kernel(tmx_problem* h, int kernel, int precision, int r
       *bytes += 2.0 * sz * (double)h->nx * (double)h->ny - sz * (double)nv;
     // the coarse stream: correction read (4) or restricted residual written (6)
     if (kernel == 4 || kernel == 6)
-      *bytes += 2.0 * sz * (double)(h->nx / 2 + 1) * (double)(h->ny / 2 + 1);
+      *bytes += 2.0 * sz * (double)h->el.levels_[1].nn;
     // direction update + operator per vertex: p_old (2 doubles), z (2 floats), xi, x read and
     // written, p and q written: 96 B
     if (kernel == 5) *bytes = 96.0 * (double)nv;

@@ -378,7 +378,9 @@ class Hierarchy {
   int au_record(int which, hipStream_t s);  // which: 0 before, 1 after the launch
   // sum of the recorded launches' durations (us) and their count since the last read
   int au_read(double* total_us, int* launches);
-  bool pair_post_ok(int l = 0) const;  // level l has even sides and a nested level below it
+  // the finest level has one below it, to which the paired kernels can restrict and from which
+  // they can prolong
+  bool pair_post_ok() const { return levels_.size() >= 2; }
   int tail_nodes_ = kTailNodes;  // largest 9-point level handled by the tail kernel
   void find_tail();
   int tail_ = -1;               // first level handled by the one-workgroup tail kernel

@@ -409,11 +409,6 @@ int Hierarchy::fine_cell_weights(hipStream_t s) {
   return 0;
 }
 
-bool Hierarchy::pair_post_ok(int l) const {
-  return l >= 0 && (int)levels_.size() >= l + 2 && levels_[l + 1].nested_from_prev &&
-         !(levels_[l].nx & 1) && !(levels_[l].ny & 1);
-}
-
 int Hierarchy::update_elasticity(const double* xi, int p, double m, hipStream_t s,
                                  bool overlap) {
   TMX_TRY(join_coarse(s));  // (the previous build reads the cell weights rewritten below)
