@@ -187,14 +187,6 @@ hipError_t prolong_bilinear(int nxf, int nyf, int nxc, int nyc, unsigned fixed, 
 template <typename T, int BS>
 hipError_t stencil_op(int nx, int ny, const T* st, int op, const T* x, const T* b, T* y,
                       T omega, hipStream_t s);
-// fused bilinear transfers of a 9-point level: bc = P^T (b - A x); y = sweep(x + P e)
-template <typename T, int BS>
-hipError_t stencil_resrestrict(int nxf, int nyf, int nxc, int nyc, unsigned fixed, const T* st,
-                               const T* x, const T* b, T* bc, hipStream_t s);
-template <typename T, int BS>
-hipError_t stencil_prolong_smooth(int nxf, int nyf, int nxc, int nyc, unsigned fixed, const T* st,
-                                  const T* x, const T* ec, const T* b, T* y, T omega,
-                                  hipStream_t s);
 // Galerkin coarse stencil Ac = P^T Af P for the given transfer (nested or bilinear); with
 // stc32, also its FP32 copy
 template <int BS>

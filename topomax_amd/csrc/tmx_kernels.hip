@@ -2135,10 +2135,10 @@ template hipError_t stencil_op<float, 1>(int, int, const float*, int, const floa
 template hipError_t stencil_op<float, 2>(int, int, const float*, int, const float*, const float*,
                                          float*, float, hipStream_t);
 
-// per-node bilinear transfers (bodies of k_restrict_bilinear / k_prolong_bilinear and of the
-// tail kernel).  Branch-free: every load is issued before any is used (out-of-range and
-// non-contributing positions get zero weight at a clamped address), so a launch costs one
-// memory round trip rather than one per contributing node.
+// per-node bilinear transfers (bodies of k_restrict_bilinear / k_prolong_bilinear).
+// Branch-free: every load is issued before any is used (out-of-range and non-contributing
+// positions get zero weight at a clamped address), so a launch costs one memory round trip rather
+// than one per contributing node.
 template <typename T, int BS>
 __device__ __forceinline__ void restrict_bilinear_node(int nxf, int nyf, int nxc, int nyc,
                                                        unsigned fixed, const T* __restrict__ rf,
@@ -2188,161 +2188,6 @@ __device__ __forceinline__ void prolong_bilinear_node(int nxf, int nyf, int nxc,
 #pragma unroll
   for (int q = 0; q < BS; ++q) xf[BS * i + q] += add[q];
 }
-
-// fused: coarse node i receives P^T (b - A x) of the fine 9-point level
-template <typename T, int BS>
-__device__ __forceinline__ void s9_resrestrict_node(int nxf, int nyf, int nxc, int nyc,
-                                                    unsigned fixed, const T* __restrict__ st,
-                                                    const T* __restrict__ x,
-                                                    const T* __restrict__ b, T* __restrict__ bc,
-                                                    size_t i) {
-  const size_t nnf = (size_t)(nxf + 1) * (nyf + 1);
-  const int I = (int)(i % (nxc + 1)), J = (int)(i / (nxc + 1));
-  double acc[BS];
-#pragma unroll
-  for (int q = 0; q < BS; ++q) acc[q] = 0.0;
-  if (!node_fixed(fixed, I, J, nxc, nyc)) {
-    const bool mx = mirrored(fixed, 0, nxf), my = mirrored(fixed, 1, nyf);
-  const int px = cpos(I, nxf, nxc, mx), py = cpos(J, nyf, nyc, my);
-    for (int dy = -1; dy <= 1; ++dy) {
-      const int fy = py + dy;
-      if (fy < 0 || fy > nyf) continue;
-      const double wy = interp1_weight(fy, nyf, nyc, J, my);
-      for (int dx = -1; dx <= 1; ++dx) {
-        const int fx = px + dx;
-        if (fx < 0 || fx > nxf) continue;
-        const double w = wy * interp1_weight(fx, nxf, nxc, I, mx);
-        if (w == 0.0) continue;
-        const size_t f = (size_t)fy * (nxf + 1) + fx;
-        T r[BS];
-#pragma unroll
-        for (int q = 0; q < BS; ++q) r[q] = b[BS * f + q];
-#pragma unroll
-        for (int kk = 0; kk < 9; ++kk) {
-          const int jx = min(max(fx + kk % 3 - 1, 0), nxf), jy = min(max(fy + kk / 3 - 1, 0), nyf);
-          const size_t j = (size_t)jy * (nxf + 1) + jx;
-#pragma unroll
-          for (int a = 0; a < BS; ++a)
-#pragma unroll
-            for (int c = 0; c < BS; ++c)
-              r[a] -= st[(size_t)(kk * BS * BS + a * BS + c) * nnf + f] * x[BS * j + c];
-        }
-#pragma unroll
-        for (int q = 0; q < BS; ++q) acc[q] += w * (double)r[q];
-      }
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < BS; ++q) bc[BS * i + q] = (T)acc[q];
-}
-
-// x + P e (bilinear) at fine node (fx, fy); fixed nodes are not corrected
-template <typename T, int BS>
-__device__ __forceinline__ void corrected(int nxf, int nyf, int nxc, int nyc, unsigned fixed,
-                                          const T* __restrict__ x, const T* __restrict__ ec,
-                                          int fx, int fy, T (&out)[BS]) {
-  const size_t f = (size_t)fy * (nxf + 1) + fx;
-#pragma unroll
-  for (int q = 0; q < BS; ++q) out[q] = x[BS * f + q];
-  if (node_fixed(fixed, fx, fy, nxf, nyf)) return;
-  const Interp1 ix = interp1(fx, nxf, nxc, mirrored(fixed, 0, nxf));
-  const Interp1 iy = interp1(fy, nyf, nyc, mirrored(fixed, 1, nyf));
-  for (int bb = 0; bb < iy.n; ++bb)
-    for (int aa = 0; aa < ix.n; ++aa) {
-      const T w = (T)(ix.w[aa] * iy.w[bb]);
-      const size_t cidx = (size_t)iy.c[bb] * (nxc + 1) + ix.c[aa];
-#pragma unroll
-      for (int q = 0; q < BS; ++q) out[q] += w * ec[BS * cidx + q];
-    }
-}
-
-// fused: one Jacobi sweep of the fine 9-point level applied to x + P e
-template <typename T, int BS>
-__device__ __forceinline__ void s9_prolong_smooth_node(int nxf, int nyf, int nxc, int nyc,
-                                                       unsigned fixed, const T* __restrict__ st,
-                                                       const T* __restrict__ x,
-                                                       const T* __restrict__ ec,
-                                                       const T* __restrict__ b,
-                                                       T* __restrict__ y, T omega, size_t v) {
-  const size_t nn = (size_t)(nxf + 1) * (nyf + 1);
-  const int ix = (int)(v % (nxf + 1)), iy = (int)(v / (nxf + 1));
-  T acc[BS], xv[BS];
-#pragma unroll
-  for (int q = 0; q < BS; ++q) acc[q] = T(0);
-#pragma unroll
-  for (int kk = 0; kk < 9; ++kk) {
-    const int jx = min(max(ix + kk % 3 - 1, 0), nxf), jy = min(max(iy + kk / 3 - 1, 0), nyf);
-    T xj[BS];
-    corrected<T, BS>(nxf, nyf, nxc, nyc, fixed, x, ec, jx, jy, xj);
-    if (kk == 4) {
-#pragma unroll
-      for (int q = 0; q < BS; ++q) xv[q] = xj[q];
-    }
-#pragma unroll
-    for (int a = 0; a < BS; ++a)
-#pragma unroll
-      for (int c = 0; c < BS; ++c) acc[a] += st[(size_t)(kk * BS * BS + a * BS + c) * nn + v] * xj[c];
-  }
-  T res[BS], d[BS];
-#pragma unroll
-  for (int q = 0; q < BS; ++q) res[q] = b[BS * v + q] - acc[q];
-  if constexpr (BS == 1) {
-    d[0] = res[0] / st[(size_t)4 * nn + v];
-  } else {
-    const T a00 = st[(size_t)(16 + 0) * nn + v], a01 = st[(size_t)(16 + 1) * nn + v];
-    const T a10 = st[(size_t)(16 + 2) * nn + v], a11 = st[(size_t)(16 + 3) * nn + v];
-    const T inv = T(1) / (a00 * a11 - a01 * a10);
-    d[0] = (a11 * res[0] - a01 * res[1]) * inv;
-    d[1] = (a00 * res[1] - a10 * res[0]) * inv;
-  }
-#pragma unroll
-  for (int q = 0; q < BS; ++q) y[BS * v + q] = xv[q] + omega * d[q];
-}
-
-template <typename T, int BS>
-__global__ void k_stencil_resrestrict(int nxf, int nyf, int nxc, int nyc, unsigned fixed,
-                                      const T* __restrict__ st, const T* __restrict__ x,
-                                      const T* __restrict__ b, T* __restrict__ bc) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < (size_t)(nxc + 1) * (nyc + 1))
-    s9_resrestrict_node<T, BS>(nxf, nyf, nxc, nyc, fixed, st, x, b, bc, i);
-}
-
-template <typename T, int BS>
-__global__ void k_stencil_prolong_smooth(int nxf, int nyf, int nxc, int nyc, unsigned fixed,
-                                         const T* __restrict__ st, const T* __restrict__ x,
-                                         const T* __restrict__ ec, const T* __restrict__ b,
-                                         T* __restrict__ y, T omega) {
-  const size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (v < (size_t)(nxf + 1) * (nyf + 1))
-    s9_prolong_smooth_node<T, BS>(nxf, nyf, nxc, nyc, fixed, st, x, ec, b, y, omega, v);
-}
-
-template <typename T, int BS>
-hipError_t stencil_resrestrict(int nxf, int nyf, int nxc, int nyc, unsigned fixed, const T* st,
-                               const T* x, const T* b, T* bc, hipStream_t s) {
-  k_stencil_resrestrict<T, BS><<<grid1d((size_t)(nxc + 1) * (nyc + 1), 64), 64, 0, s>>>(
-      nxf, nyf, nxc, nyc, fixed, st, x, b, bc);
-  return hipGetLastError();
-}
-template <typename T, int BS>
-hipError_t stencil_prolong_smooth(int nxf, int nyf, int nxc, int nyc, unsigned fixed, const T* st,
-                                  const T* x, const T* ec, const T* b, T* y, T omega,
-                                  hipStream_t s) {
-  k_stencil_prolong_smooth<T, BS><<<grid1d((size_t)(nxf + 1) * (nyf + 1), 64), 64, 0, s>>>(
-      nxf, nyf, nxc, nyc, fixed, st, x, ec, b, y, omega);
-  return hipGetLastError();
-}
-#define TMX_INST_S9F(T, BS)                                                                       \
-  template hipError_t stencil_resrestrict<T, BS>(int, int, int, int, unsigned, const T*, const T*, \
-                                                 const T*, T*, hipStream_t);                       \
-  template hipError_t stencil_prolong_smooth<T, BS>(int, int, int, int, unsigned, const T*,        \
-                                                    const T*, const T*, const T*, T*, T,           \
-                                                    hipStream_t);
-TMX_INST_S9F(double, 1)
-TMX_INST_S9F(double, 2)
-TMX_INST_S9F(float, 1)
-TMX_INST_S9F(float, 2)
 
 // ---------------------------------------------------------------- tail V-cycle
 // The bottom of the hierarchy (levels with explicit 9-point rows of at most kTailNodes nodes,

@@ -850,20 +850,12 @@ int Hierarchy::vcycle(int l, const T* b, T* out, hipStream_t s, RedSlot* dot_bz,
                         true, sweep_omega(kpre, npre)));
     w ^= 1;
   }
-  // (9-point levels keep separate residual / restriction / prolongation launches: recomputing
-  // the fine residuals per coarse node costs more than the extra launch there)
-  const bool fused_st = false;
+  // (9-point levels take separate residual / restriction / prolongation launches here: recomputing
+  // the fine residuals per coarse node costs more than the extra launch)
   if (pair_rr) {
     // done by the pair
   } else if (fused_el) {
     TMX_TRY(level_op<T>(*this, l, kResidualRestrict, buf[w], b, cb, nullptr, s));
-  } else if (fused_st) {
-    if (bs_ == 2)
-      TMX_HIP((stencil_resrestrict<T, 2>(L.nx, L.ny, C.nx, C.ny, fixed_, PrecBufs<T>::st(L),
-                                         buf[w], b, cb, s)));
-    else
-      TMX_HIP((stencil_resrestrict<T, 1>(L.nx, L.ny, C.nx, C.ny, fixed_, PrecBufs<T>::st(L),
-                                         buf[w], b, cb, s)));
   } else {
     T* r = PrecBufs<T>::r(L);
     TMX_TRY(level_op<T>(*this, l, kResidual, buf[w], b, r, nullptr, s));
@@ -884,15 +876,6 @@ int Hierarchy::vcycle(int l, const T* b, T* out, hipStream_t s, RedSlot* dot_bz,
     ex.ec = cx;
     TMX_TRY(level_op<T>(*this, l, kProlongSmooth, buf[w], b, buf[w ^ 1],
                         post == 1 ? last_dot : nullptr, s, ex, true, sweep_omega(j++, npost)));
-    w ^= 1;
-    --post;
-  } else if (fused_st) {
-    if (bs_ == 2)
-      TMX_HIP((stencil_prolong_smooth<T, 2>(L.nx, L.ny, C.nx, C.ny, fixed_, PrecBufs<T>::st(L),
-                                            buf[w], cx, b, buf[w ^ 1], (T)omega_, s)));
-    else
-      TMX_HIP((stencil_prolong_smooth<T, 1>(L.nx, L.ny, C.nx, C.ny, fixed_, PrecBufs<T>::st(L),
-                                            buf[w], cx, b, buf[w ^ 1], (T)omega_, s)));
     w ^= 1;
     --post;
   } else {
