@@ -2634,9 +2634,9 @@ hipError_t tail_vcycle(const TailDesc<T>& d0, hipStream_t s) {
     d.dense_off = (int)lds;
     lds += need;
   }
+  static_assert(kTailLdsMax <= kLdsPerCu, "one workgroup per CU");
   if (lds > 64 * 1024 && !active_recorder()) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tail_vcycle<T, BS>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const hipError_t e = raise_dyn_lds(reinterpret_cast<const void*>(&k_tail_vcycle<T, BS>));
     if (e != hipSuccess) return e;
   }
   TMX_LAUNCH_OR_RECORD(kTailWg, (tail_vcycle_body<T, BS>), 1 + 8 * kTailHelpers, lds, s,
@@ -2984,14 +2984,12 @@ hipError_t dense_invert(int n, double* a, double* /*work*/, hipStream_t s) {
   }
   // the matrix in LDS up to 160 KiB (n <= 144 unknowns; a 64-node coarsest elasticity level
   // has 128); larger ones stream it from global memory
-  constexpr size_t kLdsMax = 160 * 1024;
   const size_t lds = sizeof(double) * ((size_t)n * n + n);
-  if (lds > 64 * 1024 && lds <= kLdsMax) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_dense_invert_lds),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (lds > 64 * 1024 && lds <= kLdsPerCu) {
+    const hipError_t e = raise_dyn_lds(reinterpret_cast<const void*>(&k_dense_invert_lds));
     if (e != hipSuccess) return e;
   }
-  if (lds <= kLdsMax) TMX_LAUNCH_OR_RECORD(1024, (dense_invert_lds_body), 1, lds, s, (k_dense_invert_lds), n, a);
+  if (lds <= kLdsPerCu) TMX_LAUNCH_OR_RECORD(1024, (dense_invert_lds_body), 1, lds, s, (k_dense_invert_lds), n, a);
   else TMX_LAUNCH_OR_RECORD(1024, (dense_invert_body), 1, sizeof(double) * n, s, (k_dense_invert), n, a);
   return hipGetLastError();
 }

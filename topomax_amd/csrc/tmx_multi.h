@@ -65,11 +65,23 @@ __global__ __launch_bounds__(NT) void k_multi(const Tup* __restrict__ recs, Mult
 using MultiFn = hipError_t (*)(const void* recs, MultiMap m, unsigned grid, size_t lds,
                                hipStream_t s);
 
+// Dynamic LDS beyond 64 KiB needs the kernel's attribute raised.  The attribute is the kernel's,
+// not the launch's, and threads with handles of other sizes raise it too: so always to all that
+// the CU has beside the kernel's static LDS, never to one launch's need, which another launch
+// may exceed.
+constexpr size_t kLdsPerCu = 160 * 1024;
+inline hipError_t raise_dyn_lds(const void* kernel, size_t static_lds = 0) {
+  return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)(kLdsPerCu - static_lds));
+}
+
 template <int NT, typename Tup, auto Body>
 hipError_t multi_launch(const void* recs, MultiMap m, unsigned grid, size_t lds, hipStream_t s) {
-  if (lds > 64 * 1024) {  // (dynamic LDS beyond 64 KiB needs the kernel's attribute raised)
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_multi<NT, Tup, Body>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (lds > 64 * 1024) {
+    const void* f = reinterpret_cast<const void*>(&k_multi<NT, Tup, Body>);
+    hipFuncAttributes a;
+    hipError_t e = hipFuncGetAttributes(&a, f);
+    if (e == hipSuccess) e = raise_dyn_lds(f, a.sharedSizeBytes);
     if (e != hipSuccess) return e;
   }
   k_multi<NT, Tup, Body><<<grid, NT, lds, s>>>(static_cast<const Tup*>(recs), m);
