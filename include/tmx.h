@@ -216,7 +216,8 @@ enum tmx_option {
   TMX_OPT_CHEB_RATIO = 12,      /* smoothing band [lambda / ratio, lambda] (both; 8) */
   TMX_OPT_BAND = 13,            /* first level (>= 1) of the tiled multi-sweep V-cycle kernels
                                    (both families and precisions; default 1, FP64 elasticity
-                                   2), 0: one launch per sweep / transfer instead */
+                                   2 where level 1 has more than 200,000 nodes), 0: one launch
+                                   per sweep / transfer instead */
   TMX_OPT_BAND_FINE_FILTER = 14, /* 1 (default): the filter's finest level in the tiled
                                    kernels too */
   TMX_OPT_FINE_CELL_WEIGHTS = 15, /* elasticity finest-level V-cycle sweeps read per-cell

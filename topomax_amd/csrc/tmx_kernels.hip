@@ -2199,9 +2199,9 @@ __device__ __forceinline__ void prolong_bilinear_node(int nxf, int nyf, int nxc,
 // no range checks; the 1-D transfer weights (0, 1/2, 1) follow from a node's parity; and steps that
 // touch only the thread's own node (restriction's result and the first sweep from zero) share a
 // phase.  Per V-cycle of 816 + 225 + 65 nodes and 42 coarsest unknowns, three sweeps each way
-// (N=1000): 18.5 us in FP32 and 25.4 in FP64, before 25.0 and 52.4 (rows re-read per sweep in
-// FP64, neighbours clamped); 546 nodes and 110 unknowns (333 x 111 cells) 12.9 and 17.4, before
-// 18.0 and 36.7.  A sweep takes 0.26 us, 0.5 with two nodes a thread, the rows' load 2.3 us (FP32)
+// (N=1000): 19.4 us in FP32 and 26.1 in FP64, before 25.0 and 52.4 (rows re-read per sweep in
+// FP64, neighbours clamped); 645 nodes and 120 unknowns (333 x 111 cells) 13.8 and 18.3, before
+// 18.0 and 36.7 (about 1 us of it for the side that an odd level's single cell is on).  A sweep takes 0.26 us, 0.5 with two nodes a thread, the rows' load 2.3 us (FP32)
 // to 4.8 us (FP64).
 
 size_t tail_level_elems(int nx, int ny, int bs) {

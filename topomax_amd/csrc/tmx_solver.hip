@@ -724,11 +724,13 @@ static bool band_level(const Hierarchy& h, int l, BandLevel<T>& B) {
     // 8 x 8 tiles: 78 (399 x 133 cells, FP64) 2451 -> 2473, 45 (201 x 67 and 333 x 111 below
     // level 1) 2060 -> 2072; 105 (450 x 151) 2760 -> 2702.
     // A cell-weight level gains from the same tiles, on which a node's row is built once instead
-    // of once per sweep (640 x 320 cells: FP64 2962 -> 2849, mixed 2632 -> 2594; 1440 x 240 FP64
-    // 4122 -> 3911; 1600 x 560 4099 -> 3999 and 3296 -> 3173; 3000 x 1000 FP64 8838 -> 8617), up
-    // to 2000 of them, from where the halo counts (3948: mixed 6950 -> 7156), and in FP64, where
-    // two workgroups fit a CU, unless the second round of workgroups is half empty (646: 3174 ->
-    // 3224 with 1200 x 400 cells).
+    // of once per sweep, up to 2000 of them, from where the halo counts, and in FP64, where two
+    // workgroups fit a CU, unless the second round of workgroups is half empty.  Whole steps to
+    // 1e-8 in us with level 1's (or, marked ', level 2's) tiles as below -> these, by their count:
+    // FP64 240 2447 -> 2343, 336 2520 -> 2528, 512 2545 -> 2440; 540 3256 -> 3237, 595 the same,
+    // 646 3422 -> 3453, 741 3652 -> 3603; 820 3247 -> 3199, 1008 3225 -> 3161, 1764' 14529 -> 14386;
+    // mixed 240 2138 -> 2129, 646 2762 -> 2730, 1248 3112 -> 3052, 1456 3294 -> 3265, 1620
+    // 3551 -> 3569, 1980 5142 -> 5184; 2240 5713 -> 5659, 2584 4725 -> 4814, 3990 7733 -> 7895.
     const int nu = std::max(B.nu_down, B.nu_up), n = band_tiles(L.nx, L.ny, 16, 12);
     if (band_ext(16, nu, true) * band_ext(12, nu, true) <= (size_t)kBandThreadsMid &&
         band_lds_bytes(16, 12, nu, h.bs_, sizeof(T), B.src, true) <= kBandLdsBytes &&
